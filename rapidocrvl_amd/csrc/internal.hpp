@@ -235,6 +235,9 @@ int row_usum(hipStream_t s, int qtype, const uint8_t *src, int row_bytes, int ro
 // the small MFMA GEMM over at most 16 rows (digit planes of 16 rows)
 bool gemm_small_ok(int rows, int K);
 int gemm_small_rows(hipStream_t s, int qtype, int nmat, const GemmParams &p, int epi);
+// a layer matrix of the batched decode step over operand images (rows.hip)
+struct RowsParams;
+int rows_gemm(hipStream_t s, int qtype, int epi, const RowsParams &p);
 // vision projector (projector.hip); callers hold the context lock
 int project_locked(pocr_projector *p, int grid_t, int grid_h, int grid_w, int *rows);
 int project_upload_locked(pocr_projector *p, const float *vision_rows, int grid_t, int grid_h, int grid_w,

@@ -1267,6 +1267,49 @@ static __global__ void __launch_bounds__(kThreads) k_rope(float *q, float *k, co
     }
 }
 
+// ---------------------------------------------------------------------------
+// Operand images of a batched decode step (rows.hpp): activation rows as three
+// bf16 planes in the order the matrix kernels read them.
+// ---------------------------------------------------------------------------
+// bytes of the operand image of K columns
+__host__ __device__ constexpr size_t rows_image_bytes(int K) { return (size_t)K * 16 * 3 * 2; }
+
+struct Planes3 {
+    uint16_t p[3];
+};
+__device__ __forceinline__ Planes3 split_planes(float x) {
+    Planes3 r;
+    const __bf16 hi = (__bf16)x;
+    const float r1 = x - (float)hi;  // exact: the low 16 bits
+    const __bf16 mid = (__bf16)r1;
+    const __bf16 lo = (__bf16)(r1 - (float)mid);
+    r.p[0] = __builtin_bit_cast(uint16_t, hi);
+    r.p[1] = __builtin_bit_cast(uint16_t, mid);
+    r.p[2] = __builtin_bit_cast(uint16_t, lo);
+    return r;
+}
+
+// element index of (row n, column k, plane) in an operand image
+__device__ __forceinline__ size_t rows_at(bool pack, int n, int k, int pl) {
+    const int u = k >> 7, lg = (k >> 5) & 3, j = (k >> 3) & 3;
+    const int group = pack ? (u * 4 + j) * 64 + 3 * n + pl + 16 * lg : ((u * 3 + pl) * 4 + j) * 64 + n + 16 * lg;
+    return (size_t)group * 8 + (k & 7);
+}
+
+__device__ __forceinline__ void rows_put(uint16_t *img, bool pack, int n, int k, float x) {
+    const Planes3 s = split_planes(x);
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) img[rows_at(pack, n, k, pl)] = s.p[pl];
+}
+// columns k..k+3 (k a multiple of 4)
+__device__ __forceinline__ void rows_put4(uint16_t *img, bool pack, int n, int k, const float4 &x) {
+    const Planes3 a = split_planes(x.x), b = split_planes(x.y), c = split_planes(x.z), d = split_planes(x.w);
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl)
+        *reinterpret_cast<uint2 *>(img + rows_at(pack, n, k, pl)) =
+            make_uint2(a.p[pl] | ((uint32_t)b.p[pl] << 16), c.p[pl] | ((uint32_t)d.p[pl] << 16));
+}
+
 // Step prologue: token/position bookkeeping, RoPE table (buildMRoPETable,
 // model.go:7318-7357: f64 angle, f64 cos/sin rounded to f32), embedding row.
 // mode 0: h and pos were written by the host.  mode 1: greedy decode — the
@@ -1277,10 +1320,12 @@ static __global__ void __launch_bounds__(kThreads) k_rope(float *q, float *k, co
 // and the table entry is computed while the slots are reduced; the token's
 // embedding row is requested while thread 0 settles the state.  Results are
 // stored only once the step is known to go ahead.
+// put(i, j, x) takes the row: column i = t + j·kThreads (mode 1).
 constexpr int kStepEmb = 4;  // embedding floats a thread holds across the state barrier
-__device__ __forceinline__ void step_begin_body(StepState *st, const float *embed, float *h, int hidden, int vocab,
+template <class Put>
+__device__ __forceinline__ void step_begin_body(StepState *st, const float *embed, int hidden, int vocab,
                                                 const double *freq, const uint8_t *axis, int mode, int32_t *tokens,
-                                                int max_tokens) {
+                                                int max_tokens, Put &&put) {
     __shared__ int s_err;
     __shared__ unsigned long long s_key;
     const int t = threadIdx.x;
@@ -1381,17 +1426,18 @@ __device__ __forceinline__ void step_begin_body(StepState *st, const float *embe
 #pragma unroll
         for (int j = 0; j < kStepEmb; ++j) {
             const int i = t + j * kThreads;
-            if (i < hidden) h[i] = e[j];
+            if (i < hidden) put(i, j, e[j]);
         }
         const float *src = embed + (size_t)tok * hidden;
-        for (int i = t + kStepEmb * kThreads; i < hidden; i += kThreads) h[i] = src[i];
+        for (int i = t + kStepEmb * kThreads, j = kStepEmb; i < hidden; i += kThreads, ++j) put(i, j, src[i]);
     }
 }
 
 static __global__ void __launch_bounds__(kThreads) k_step_begin(StepState *st, const float *embed, float *h, int hidden,
                                                            int vocab, const double *freq, const uint8_t *axis,
                                                            int mode, int32_t *tokens, int max_tokens) {
-    step_begin_body(st, embed, h, hidden, vocab, freq, axis, mode, tokens, max_tokens);
+    step_begin_body(st, embed, hidden, vocab, freq, axis, mode, tokens, max_tokens,
+                    [&](int i, int, float x) { h[i] = x; });
 }
 
 // Greedy decode of several sequences in one step: workgroup b runs sequence
@@ -1407,13 +1453,30 @@ struct StepBatch {
 typedef __attribute__((address_space(4))) const StepBatch KernargStepBatch;
 static __global__ void __launch_bounds__(kThreads) k_step_begin_multi(StepBatch b, const float *embed, float *h,
                                                                  int hidden, int vocab, const double *freq,
-                                                                 const uint8_t *axis) {
+                                                                 const uint8_t *axis, const float *norm_w,
+                                                                 uint16_t *img, int pack, float *ssq) {
     (void)b;
 #if defined(__HIP_DEVICE_COMPILE__)
+    __shared__ float red[kWaves];
     const KernargStepBatch *kb = (KernargStepBatch *)__builtin_amdgcn_kernarg_segment_ptr();
     const int i = blockIdx.x;
-    step_begin_body(kb->st[i], embed, h + (size_t)i * hidden, hidden, vocab, freq, axis, 1, kb->tokens[i],
-                    kb->max_tokens[i]);
+    float *row = h + (size_t)i * hidden;
+    // with images, the first layer's operand too: the row times its norm
+    // weight (requested here, ahead of the token's row), and Σx²
+    float nw[kStepEmb];
+#pragma unroll
+    for (int j = 0; j < kStepEmb; ++j) nw[j] = img ? norm_w[min((int)threadIdx.x + j * kThreads, hidden - 1)] : 0.0f;
+    float s = 0.0f;
+    step_begin_body(kb->st[i], embed, hidden, vocab, freq, axis, 1, kb->tokens[i], kb->max_tokens[i],
+                    [&](int c, int j, float x) {
+                        row[c] = x;
+                        if (!img) return;  // uniform
+                        s = fmaf(x, x, s);
+                        rows_put(img, pack != 0, i, c, x * (j < kStepEmb ? nw[j < kStepEmb ? j : 0] : norm_w[c]));
+                    });
+    if (!img) return;
+    s = block_sum(s, red);
+    if (threadIdx.x == 0) ssq[i] = s;
 #endif
 }
 
@@ -1462,6 +1525,9 @@ struct AttnParams {
     int rows_cap;          // rows the splits are cut from (cache capacity)
     float scale;
     int chunk;             // rows per split, attn_chunk(rows_cap, nsplit, 4·RPW)
+    int img_row;           // this sequence's row of img
+    int img_pack;          // img columns are (row, plane) pairs
+    uint16_t *img;         // null, or the operand image the merge writes in place of head_out
 };
 
 // rows per split: the capacity's share rounded up to 16, at most max_chunk
@@ -1868,8 +1934,13 @@ __device__ __forceinline__ bool attn_merge_body(AttnParams p, float *dst = nullp
             r.w += a.w;
         }
         const float inv = 1.0f / l_lds;
-        float *o = dst ? dst : p.head_out + (size_t)hq * kHD;
-        *reinterpret_cast<float4 *>(o + 4 * t) = make_float4(r.x * inv, r.y * inv, r.z * inv, r.w * inv);
+        const float4 v = make_float4(r.x * inv, r.y * inv, r.z * inv, r.w * inv);
+        if (p.img) {  // uniform
+            rows_put4(p.img, p.img_pack != 0, p.img_row, hq * kHD + 4 * t, v);
+        } else {
+            float *o = dst ? dst : p.head_out + (size_t)hq * kHD;
+            *reinterpret_cast<float4 *>(o + 4 * t) = v;
+        }
     }
     return true;
 }

@@ -10,6 +10,7 @@
 #include "gemm.hpp"
 #include "vnni.hpp"
 #include "head.hpp"
+#include "rows.hpp"
 #include "internal.hpp"
 
 namespace pocr {
@@ -2753,13 +2754,19 @@ struct DecodeBatch {
     pocr_seq *seq[kMaxBatch] = {};
     float *h = nullptr, *v = nullptr, *qkv = nullptr, *ho = nullptr, *g = nullptr;
     StepState *pad = nullptr;  // step state of the padding vectors
-    // digit planes of 16 rows, row scales and sums (the wide step, n > 4, and
-    // the wide LM head from kBatchWideHeadMin rows), and the wide step's row
-    // step states (the o_proj epilogue reads each sequence's clen)
+    // digit planes of 16 rows, row scales and sums of the LM head (from
+    // kBatchWideHeadMin rows), and the rows' step states (the o_proj epilogue
+    // reads each sequence's clen)
     int8_t *xd = nullptr;
     float *xs = nullptr;
     int *xb = nullptr;
     StepState **rst = nullptr;
+    // operand images of the matrix kernels (batch_rows_ok): the normed hidden
+    // rows, the attention output and the SwiGLU output, one allocation; and the
+    // partial Σx² of the hidden rows
+    uint16_t *img = nullptr;
+    float *ssq = nullptr;
+    bool rows_ok[2] = {false, false};  // more than kMaxNV rows, at most
     float *logits = nullptr;  // [16][vocab] greedy rows of the MFMA LM head (vocab a multiple of 16)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -2769,7 +2776,7 @@ struct DecodeBatch {
         if (graph) (void)hipGraphDestroy(graph);
         if (owns)
             for (void *p : {(void *)h, (void *)v, (void *)qkv, (void *)ho, (void *)g, (void *)pad, (void *)xd,
-                            (void *)xs, (void *)xb, (void *)rst, (void *)logits})
+                            (void *)xs, (void *)xb, (void *)rst, (void *)img, (void *)ssq, (void *)logits})
                 if (p) (void)hipFree(p);
     }
     StepState *st(int i) const { return i < n ? seq[i]->st : pad; }
@@ -2838,29 +2845,25 @@ GemmParams batch_gemm(const DecodeBatch &b, const pocr_weight *w, int K) {
     return p;
 }
 
-// One layer of the wide step (5..16 sequences): digit planes of the rows,
-// then the small MFMA GEMM with the prefill epilogues (each row a sequence);
-// attention and its merge as in the narrow step.
-int batch_layer_wide(DecodeBatch &b, const LayerW &L, int li, bool last, int rpw, int max_split) {
-    pocr_model *m = b.m;
-    const pocr_config &c = m->cfg;
-    hipStream_t st = m->ctx->stream;
-    const int H = c.hidden, Q = c.heads * c.head_dim, KV = c.kv_heads * c.head_dim, F = c.intermediate;
-    const int QKV = Q + 2 * KV;
-    const int qt = L.w[POCR_W_Q]->qtype;
-    // 1. RMSNorm(h)·ln1 → q|k|v
-    RC(batch_digitize(b, qt, b.h, H, L.ln1));
-    GemmParams g = batch_gemm(b, L.w[POCR_W_Q], H);
-    g.m[1] = dev_mat(L.w[POCR_W_K]);
-    g.m[2] = dev_mat(L.w[POCR_W_V]);
-    g.seg_end[0] = Q;
-    g.seg_end[1] = Q + KV;
-    g.seg_end[2] = QKV;
-    g.rows = QKV;
-    g.out = b.qkv;
-    g.out_stride = QKV;
-    RC(gemm_small_rows(st, qt, 1, g, G_PLAIN));
-    // 2. RoPE + KV append + split attention, then the merge
+// The layers' weights all have tile images, the matrix kernels' only demand
+// (rows a multiple of 16, columns of 128).  Up to kMaxNV rows the shapes of the
+// streaming GEMV are asked for besides: the LM head's passes need them there,
+// and a step that takes other shapes is refused as a whole.
+bool batch_rows_ok(const pocr_model *m, bool narrow) {
+    for (const LayerW &L : m->layers) {
+        for (const pocr_weight *w : L.w)
+            if (!w || !w->tiled || (narrow && !gemv_fast_shape(dev_mat(w)))) return false;
+        if (L.w[POCR_W_Q]->qtype != L.w[POCR_W_K]->qtype || L.w[POCR_W_Q]->qtype != L.w[POCR_W_V]->qtype ||
+            L.w[POCR_W_GATE]->qtype != L.w[POCR_W_UP]->qtype)
+            return false;
+    }
+    return m->cfg.head_dim == kHD;
+}
+
+// the batch's attention arguments of layer li
+AttnMulti batch_attn(const DecodeBatch &b, int li, int rpw, bool images) {
+    const pocr_config &c = b.m->cfg;
+    const int Q = c.heads * c.head_dim, KV = c.kv_heads * c.head_dim, QKV = Q + 2 * KV;
     AttnMulti am{};
     for (int i = 0; i < b.n; ++i) {
         pocr_seq *s = b.seq[i];
@@ -2877,36 +2880,82 @@ int batch_layer_wide(DecodeBatch &b, const LayerW &L, int li, bool last, int rpw
         a.kvh = c.kv_heads;
         attn_shape(a, s->cap, rpw);
         a.scale = (float)(1.0 / std::sqrt((double)c.head_dim));
+        if (images) {
+            a.img = b.img + rows_image_bytes(c.hidden) / 2;
+            a.img_row = i;
+            a.img_pack = b.n <= kRowsPackMax;
+        }
     }
+    return am;
+}
+
+int batch_attention(const DecodeBatch &b, const AttnMulti &am, int rpw, int max_split) {
+    const pocr_config &c = b.m->cfg;
+    hipStream_t st = b.m->ctx->stream;
     const dim3 ag(c.kv_heads, max_split, b.n);
     if (rpw == 8) hipLaunchKernelGGL(k_attn_decode_multi<8>, ag, dim3(kThreads), 0, st, am);
     else hipLaunchKernelGGL(k_attn_decode_multi<16>, ag, dim3(kThreads), 0, st, am);
     launch_attn_merge_multi(st, dim3(c.heads, 1, b.n), max_split, am);
     HIP_TRY(hipGetLastError());
-    // 3. o_proj + residual (+ the Q4/Q6 behaviour by each sequence's clen)
+    return POCR_OK;
+}
+
+// One layer over operand images: q|k|v, attention, its merge, o_proj, gate/up
+// and down, each writing the next one's operand.  li = 0 reads what the step
+// prologue wrote.
+int batch_layer_rows(const DecodeBatch &b, int li, int rpw, int max_split) {
+    pocr_model *m = b.m;
+    const pocr_config &c = m->cfg;
+    hipStream_t st = m->ctx->stream;
+    const LayerW &L = m->layers[li];
+    const bool last = li + 1 == c.layers;
+    const int H = c.hidden, Q = c.heads * c.head_dim, KV = c.kv_heads * c.head_dim, F = c.intermediate;
+    uint16_t *img_h = b.img, *img_o = img_h + rows_image_bytes(H) / 2, *img_g = img_o + rows_image_bytes(Q) / 2;
+    auto params = [&](std::initializer_list<int> roles, int rows, int K, const uint16_t *x) {
+        RowsParams p{};
+        int i = 0;
+        for (const int role : roles) {
+            p.w[i] = L.w[role]->tiled;
+            p.scale[i++] = L.w[role]->scale;
+        }
+        p.seg_end[0] = p.seg_end[1] = rows;
+        p.rows = rows;
+        p.nst = K / kStageCols;
+        p.ntok = b.n;
+        p.x = x;
+        p.eps = c.rms_norm_eps;
+        return p;
+    };
+    RowsParams q = params({POCR_W_Q, POCR_W_K, POCR_W_V}, Q + 2 * KV, H, img_h);
+    q.seg_end[0] = Q;
+    q.seg_end[1] = Q + KV;
+    q.ssq = b.ssq;
+    q.nparts = li == 0 ? 1 : H / 16;
+    q.out = b.qkv;
+    RC(rows_gemm(st, L.w[POCR_W_Q]->qtype, R_PLAIN, q));
+    RC(batch_attention(b, batch_attn(b, li, rpw, true), rpw, max_split));
     const pocr_weight *wo = L.w[POCR_W_O];
-    RC(batch_digitize(b, wo->qtype, b.ho, Q, nullptr));
-    GemmParams o = batch_gemm(b, wo, Q);
+    RowsParams o = params({POCR_W_O}, H, Q, img_o);
     o.h = b.h;
-    o.vbuf = b.v;
+    o.norm_w = L.ln2;
+    o.img = img_h;
+    o.ssq_out = b.ssq;
+    o.rst = b.rst;
     o.quirk = (m->quirk && (wo->qtype == POCR_Q4 || wo->qtype == POCR_Q6)) ? 1 : 0;
-    RC(gemm_small_rows(st, wo->qtype, 1, o, G_OPROJ));
-    // 4. RMSNorm(v)·ln2 → gate/up → SiLU(g)·u
-    const pocr_weight *wg = L.w[POCR_W_GATE];
-    RC(batch_digitize(b, wg->qtype, b.v, H, L.ln2));
-    GemmParams gu = batch_gemm(b, wg, H);
-    gu.m[1] = dev_mat(L.w[POCR_W_UP]);
-    gu.out = b.g;
-    gu.out_stride = F;
-    RC(gemm_small_rows(st, wg->qtype, 2, gu, G_SWIGLU));
-    // 5. down + residual; last layer: v = h + down
-    const pocr_weight *wd = L.w[POCR_W_DOWN];
-    RC(batch_digitize(b, wd->qtype, b.g, F, nullptr));
-    GemmParams d = batch_gemm(b, wd, F);
+    RC(rows_gemm(st, wo->qtype, R_OPROJ, o));
+    RowsParams gu = params({POCR_W_GATE, POCR_W_UP}, F, H, img_h);
+    gu.ssq = b.ssq;
+    gu.nparts = H / 16;
+    gu.img = img_g;
+    RC(rows_gemm(st, L.w[POCR_W_GATE]->qtype, R_SWIGLU, gu));
+    RowsParams d = params({POCR_W_DOWN}, H, F, img_g);
     d.h = b.h;
     d.vbuf = b.v;
     d.last = last ? 1 : 0;
-    return gemm_small_rows(st, wd->qtype, 1, d, G_DOWN);
+    d.norm_w = last ? m->final_norm : m->layers[li + 1].ln1;
+    d.img = img_h;
+    d.ssq_out = b.ssq;
+    return rows_gemm(st, L.w[POCR_W_DOWN]->qtype, R_DOWN, d);
 }
 
 int enqueue_batch_step(DecodeBatch &b) {
@@ -2922,8 +2971,9 @@ int enqueue_batch_step(DecodeBatch &b) {
         sb.tokens[i] = b.seq[i]->tokens;
         sb.max_tokens[i] = b.seq[i]->max_tokens;
     }
+    const bool rows = b.n > 1 && b.rows_ok[b.n <= kMaxNV];
     hipLaunchKernelGGL(k_step_begin_multi, dim3(b.n), dim3(kThreads), 0, st, sb, m->embed, b.h, H, c.vocab, m->freq,
-                       m->axis);
+                       m->axis, m->layers[0].ln1, rows ? b.img : nullptr, b.n <= kRowsPackMax ? 1 : 0, b.ssq);
     HIP_TRY(hipGetLastError());
     // one rows-per-wave for all: the largest the sequences' capacities pick
     // (no more splits than any sequence's records were sized for)
@@ -2931,11 +2981,12 @@ int enqueue_batch_step(DecodeBatch &b) {
     for (int i = 0; i < b.n; ++i) rpw = std::max(rpw, b.seq[i]->rpw);
     for (int i = 0; i < b.n; ++i) max_split = std::max(max_split, attn_nsplit(b.seq[i]->cap, rpw));
     const bool wide = b.n > kMaxNV;
+    if (wide && !rows) return fail(POCR_ERR_UNSUPPORTED, "batch step: %d rows need the weights' tile images", b.n);
     for (int li = 0; li < c.layers; ++li) {
         const LayerW &L = m->layers[li];
         const bool last = li + 1 == c.layers;
-        if (wide) {
-            RC(batch_layer_wide(b, L, li, last, rpw, max_split));
+        if (rows) {
+            RC(batch_layer_rows(b, li, rpw, max_split));
             continue;
         }
         // 1. RMSNorm(h)·ln1 → q|k|v for every sequence
@@ -2956,28 +3007,7 @@ int enqueue_batch_step(DecodeBatch &b) {
         GemvNV q = batch_nv(b, H, QKV);
         RC(gemv_launch(st, p, 1, PRO_RMSNORM, EPI_PLAIN, kBigGrid, b.nv, &q));
         // 2. per sequence: RoPE + KV append + split attention, then the merge
-        AttnMulti am{};
-        for (int i = 0; i < b.n; ++i) {
-            pocr_seq *s = b.seq[i];
-            AttnParams &a = am.a[i];
-            a.q = b.qkv + (size_t)i * QKV;
-            a.k_new = a.q + Q;
-            a.v_new = a.q + Q + KV;
-            a.kc = layer_k(s, li);
-            a.vc = layer_v(s, li);
-            a.st = s->st;
-            a.part = s->part;
-            a.head_out = b.ho + (size_t)i * Q;
-            a.heads = c.heads;
-            a.kvh = c.kv_heads;
-            attn_shape(a, s->cap, rpw);
-            a.scale = (float)(1.0 / std::sqrt((double)c.head_dim));
-        }
-        const dim3 ag(c.kv_heads, max_split, b.n);
-        if (rpw == 8) hipLaunchKernelGGL(k_attn_decode_multi<8>, ag, dim3(kThreads), 0, st, am);
-        else hipLaunchKernelGGL(k_attn_decode_multi<16>, ag, dim3(kThreads), 0, st, am);
-        launch_attn_merge_multi(st, dim3(c.heads, 1, b.n), max_split, am);
-        HIP_TRY(hipGetLastError());
+        RC(batch_attention(b, batch_attn(b, li, rpw, false), rpw, max_split));
         // 3. o_proj + residual (+ the Q4/Q6 behaviour per sequence)
         const pocr_weight *wo = L.w[POCR_W_O];
         GemvParams o = gemv_params_1(wo);
@@ -3070,8 +3100,9 @@ int32_t pending_token(const StepState &hs) {
     return (int32_t)(0xFFFFFFFFu - (uint32_t)(argmax_of(hs) & 0xFFFFFFFFull));
 }
 
-// vector buffers for b.cap rows; from kBatchWideHeadMin rows also digit planes
-// (16 rows of the widest input), with cap > 4 the wide step's row-state table
+// vector buffers for b.cap rows; from kBatchWideHeadMin rows also the LM head's
+// digit planes (16 rows of the widest input); the operand images and row states
+// of batch_layer_rows
 int batch_alloc(DecodeBatch &b) {
     const pocr_config &c = b.m->cfg;
     const size_t H = c.hidden, Q = (size_t)c.heads * c.head_dim, KV = (size_t)c.kv_heads * c.head_dim;
@@ -3092,16 +3123,26 @@ int batch_alloc(DecodeBatch &b) {
         HIP_TRY(hipMalloc(&b.xs, 16 * sizeof(float)));
         HIP_TRY(hipMalloc(&b.xb, 16 * 4 * sizeof(int)));
     }
+    b.rows_ok[0] = batch_rows_ok(b.m, false);
+    b.rows_ok[1] = batch_rows_ok(b.m, true);
+    if (b.rows_ok[0] || rows > (size_t)kMaxNV) HIP_TRY(hipMalloc(&b.rst, kMaxBatch * sizeof(StepState *)));
+    if (b.rows_ok[0]) {
+        // zeros: a row whose first step stops at once never writes its column
+        const size_t img = rows_image_bytes((int)(H + Q) + c.intermediate), ssq = (H / 16) * 16 * sizeof(float);
+        HIP_TRY(hipMalloc(&b.img, img));
+        HIP_TRY(hipMemsetAsync(b.img, 0, img, s));
+        HIP_TRY(hipMalloc(&b.ssq, ssq));
+        HIP_TRY(hipMemsetAsync(b.ssq, 0, ssq, s));
+    }
     if (rows > (size_t)kMaxNV) {
-        HIP_TRY(hipMalloc(&b.rst, kMaxBatch * sizeof(StepState *)));
         if (gemm_small_ok(c.vocab, c.hidden)) HIP_TRY(hipMalloc(&b.logits, (size_t)16 * c.vocab * 4));
     }
     return POCR_OK;
 }
 
-// the row-state table of a wide step (rows = sequences), before its capture
+// the row-state table of a step over rows (rows = sequences), before its capture
 int batch_set_rows(DecodeBatch &b) {
-    if (b.n <= kMaxNV) return POCR_OK;
+    if (!b.rst) return POCR_OK;
     StepState *h[kMaxBatch] = {};
     for (int i = 0; i < b.n; ++i) h[i] = b.seq[i]->st;
     HIP_TRY(hipMemcpy(b.rst, h, sizeof(h), hipMemcpyHostToDevice));
@@ -3356,6 +3397,9 @@ static int batch_capture(pocr_batch *b) {
     d->xs = b->bufs.xs;
     d->xb = b->bufs.xb;
     d->rst = b->bufs.rst;
+    d->img = b->bufs.img;
+    d->ssq = b->bufs.ssq;
+    std::copy(b->bufs.rows_ok, b->bufs.rows_ok + 2, d->rows_ok);
     d->logits = b->bufs.logits;
     RC(batch_set_rows(*d));
     if (b->use_graph) {

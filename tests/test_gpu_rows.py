@@ -1,0 +1,53 @@
+"""The batched step's matrix kernels (2 to 16 rows over bf16 planes): the tokens
+and the K/V rows of a batched decode against each sequence decoded alone.  Both
+paths sum in f32 over exact products, about 1e-6 apart after three layers
+(2-norm); the bound is 2e-5."""
+import numpy as np
+import pytest
+
+from rapidocrvl_amd import lib, synth
+from rapidocrvl_amd.config import DecoderConfig
+
+pytestmark = pytest.mark.gpu
+
+Q8, Q4, Q6 = 1000, 1001, 1002
+
+
+def _cfg(hidden, inter, heads, kv_heads):
+    return DecoderConfig(hidden=hidden, inter=inter, layers=3, heads=heads, kv_heads=kv_heads, head_dim=128, vocab=1024,
+                         eps=1e-5, rope_theta=500000.0)
+
+
+ERNIE = _cfg(1024, 3072, 16, 2)
+# K of 4 and 12 stages of 128 columns: waves without a stage, and with two
+RAGGED = _cfg(512, 1536, 4, 1)
+# 4 and 10 stages; 1,280 rows of gate and up
+SMALL = _cfg(512, 1280, 4, 2)
+
+
+@pytest.mark.parametrize("cfg,qtype,nseq", [
+    (RAGGED, Q8, 2), (RAGGED, Q6, 3), (RAGGED, Q8, 4),   # (row, plane) columns
+    (SMALL, Q4, 5), (SMALL, Q6, 5),                      # their last row
+    (SMALL, Q4, 6), (SMALL, Q8, 8), (SMALL, Q6, 9),      # plane by plane; 8 rows a workgroup and the rest
+    (SMALL, Q8, 16), (ERNIE, Q4, 3), (ERNIE, Q4, 9), (ERNIE, Q6, 16), (ERNIE, Q8, 2),
+])
+def test_rows_match_single_decode(ctx, cfg, qtype, nseq):
+    m = lib.Model(ctx, cfg)
+    m.load_weights(synth.make_weights(cfg, qtype, seed=31))
+    n_new = 6
+    lens = [1 + (5 * i) % 13 for i in range(nseq)]  # 1..13: residual kept in place and not
+    prompts = [synth.prompt_ids(n, seed=300 + i, high=cfg.vocab) for i, n in enumerate(lens)]
+
+    def prefilled(ids):
+        s = m.seq(len(ids) + n_new + 4)
+        return s, int(s.generate(ids, 1, eos=(), use_prefill=True)[0])
+
+    batch, firsts = zip(*[prefilled(ids) for ids in prompts])
+    got = lib.decode_batch(list(batch), list(firsts), lens, n_new, eos=())
+    for i, ids in enumerate(prompts):
+        s, first = prefilled(ids)
+        assert list(got[i]) == list(s.decode_greedy(first, lens[i], n_new, eos=())), i
+        for li in range(cfg.layers):
+            for a, b in zip(batch[i].read_kv(li), s.read_kv(li)):
+                err = np.linalg.norm(a - b) / np.linalg.norm(b)
+                assert err < 2e-5, (i, li, err)
