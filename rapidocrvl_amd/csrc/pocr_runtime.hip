@@ -2456,12 +2456,12 @@ int pocr::launch_attn_ordered_rows(hipStream_t s, const float *qkv, int stride, 
     // 56 KB of LDS (with the q rows under 64 KB; two workgroups per CU or more)
     int hpw = 1;
     for (const int c : {8, 4, 2})
-        if (group % c == 0 && (size_t)c * rows * 4 <= 56 * 1024) {
+        if (group % c == 0 && (size_t)c * ordered_pitch(rows) * 4 <= 56 * 1024) {
             hpw = c;
             break;
         }
     const dim3 grid(kvh * (group / hpw), n);
-    const size_t lds = (size_t)hpw * rows * 4;
+    const size_t lds = (size_t)hpw * ordered_pitch(rows) * 4;
     switch (hpw) {
     case 8: hipLaunchKernelGGL(k_attn_ordered_rows<8>, grid, dim3(kThreads), lds, s, qkv, stride, kc, vc, heads, kvh, clen0, scale, out, out_stride); break;
     case 4: hipLaunchKernelGGL(k_attn_ordered_rows<4>, grid, dim3(kThreads), lds, s, qkv, stride, kc, vc, heads, kvh, clen0, scale, out, out_stride); break;
