@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -78,11 +79,15 @@ struct pocr_ctx {
     DevBuf gxd, gxs, gxb;  // batched GEMV activation digits
     DevBuf topk_part, samp;  // top-k partial keys, sampler state
     DevBuf wide;             // wide sampler buffers (pocr::WideBufs)
-    // pinned host staging for large host→device uploads: two halves, each
-    // reused once the copy recorded on its event has finished
+    // pinned host staging of large transfers: two halves, each reused once the
+    // copy recorded on its event has finished
     uint8_t *pin = nullptr;
     size_t pin_half = 0;
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
+    // pinned host memory of small transfers, each way; in_used bytes of the
+    // former belong to copies that may still run
+    uint8_t *small_in = nullptr, *small_out = nullptr;
+    size_t small_in_n = 0, small_out_n = 0, in_used = 0;
     // pinned host read-back of the greedy decode loop: the step state and the
     // tokens of one batch of steps, fetched with one synchronization
     uint8_t *readback = nullptr;
@@ -194,6 +199,20 @@ int prefill_ids_locked(pocr_seq *s, const int32_t *ids, int n, const float *imag
                        const int32_t *pos3, float *logits, int32_t *token, bool image_on_device = false);
 // host → device copy through the context's pinned staging (stream-ordered)
 int upload_staged(pocr_ctx *ctx, void *dst, const void *src, size_t bytes);
+// device → host copy through the same staging; dst holds the bytes on return,
+// and the stream's earlier work has finished
+int download_staged(pocr_ctx *ctx, void *dst, const void *src, size_t bytes);
+// Transfers of a call whose operands are host arrays: the parts go through
+// pinned memory, the small ones with one copy kernel for all of them.
+// stage_in is stream-ordered (src may be reused at once); stage_out returns
+// with the bytes in place and the stream finished.
+struct HostPart {
+    void *dst;
+    const void *src;
+    size_t bytes;  // a multiple of 4; 0: skipped
+};
+int stage_in(pocr_ctx *ctx, std::initializer_list<HostPart> parts);
+int stage_out(pocr_ctx *ctx, std::initializer_list<HostPart> parts);
 int batched_gemv(pocr_ctx *ctx, const DevMat &w, const float *x, int m, float *out);
 int read_state(pocr_seq *s, StepState *out);
 unsigned long long argmax_of(const StepState &s);

@@ -106,6 +106,20 @@ static int scratch_setup(int device, float **out) {
     return POCR_OK;
 }
 
+// an area of at least `bytes` (64 KB or a power of two; at most kCopyParts
+// parts' worth), grown with the stream idle
+static int small_area(pocr_ctx *ctx, uint8_t *&area, size_t &cap, size_t bytes) {
+    if (bytes <= cap) return POCR_OK;
+    size_t n = 64u << 10;
+    while (n < bytes) n *= 2;
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (area) (void)hipHostFree(area);
+    area = nullptr;
+    cap = 0;
+    HIP_TRY(hipHostMalloc((void **)&area, n, hipHostMallocDefault));
+    cap = n;
+    return POCR_OK;
+}
 extern "C" int pocr_ctx_create(int device, pocr_ctx **out) {
     if (!out) return fail(POCR_ERR_ARG, "pocr_ctx_create: null out");
     *out = nullptr;
@@ -127,6 +141,13 @@ extern "C" int pocr_ctx_create(int device, pocr_ctx **out) {
         delete c;
         return fail(POCR_ERR_DEVICE, "hipStreamCreate failed");
     }
+    // the first op-level call of a context would wait 25 µs for each of these
+    int rc = small_area(c, c->small_in, c->small_in_n, 1);
+    if (rc == POCR_OK) rc = small_area(c, c->small_out, c->small_out_n, 1);
+    if (rc != POCR_OK) {
+        ctx_release(c);
+        return rc;
+    }
     *out = c;
     return POCR_OK;
 }
@@ -141,6 +162,8 @@ void pocr::ctx_release(pocr_ctx *ctx) {
     for (hipEvent_t &e : ctx->pin_ev)
         if (e) (void)hipEventDestroy(e);
     if (ctx->pin) (void)hipHostFree(ctx->pin);
+    if (ctx->small_in) (void)hipHostFree(ctx->small_in);
+    if (ctx->small_out) (void)hipHostFree(ctx->small_out);
     if (ctx->readback) (void)hipHostFree(ctx->readback);
     delete ctx;
 }
@@ -148,13 +171,18 @@ void pocr::ctx_release(pocr_ctx *ctx) {
 // Chunks of at most pin_half bytes alternate between the two pinned halves:
 // the host copy into a half waits only for that half's previous transfer, so
 // the memcpy of one chunk overlaps the DMA of the one before.
-int pocr::upload_staged(pocr_ctx *ctx, void *dst, const void *src, size_t bytes) {
+static int pin_halves(pocr_ctx *ctx) {
     constexpr size_t kHalf = 2u << 20;
-    if (!ctx->pin) {
-        HIP_TRY(hipHostMalloc((void **)&ctx->pin, 2 * kHalf, hipHostMallocDefault));
-        ctx->pin_half = kHalf;
-        for (hipEvent_t &e : ctx->pin_ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
+    if (ctx->pin) return POCR_OK;
+    for (hipEvent_t &e : ctx->pin_ev)
+        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    HIP_TRY(hipHostMalloc((void **)&ctx->pin, 2 * kHalf, hipHostMallocDefault));
+    ctx->pin_half = kHalf;
+    return POCR_OK;
+}
+
+int pocr::upload_staged(pocr_ctx *ctx, void *dst, const void *src, size_t bytes) {
+    RC(pin_halves(ctx));
     const uint8_t *s8 = static_cast<const uint8_t *>(src);
     uint8_t *d8 = static_cast<uint8_t *>(dst);
     for (size_t off = 0, c = 0; off < bytes; off += ctx->pin_half, ++c) {
@@ -164,6 +192,124 @@ int pocr::upload_staged(pocr_ctx *ctx, void *dst, const void *src, size_t bytes)
         std::memcpy(half, s8 + off, len);
         HIP_TRY(hipMemcpyAsync(d8 + off, half, len, hipMemcpyHostToDevice, ctx->stream));
         HIP_TRY(hipEventRecord(ctx->pin_ev[c & 1], ctx->stream));
+    }
+    return POCR_OK;
+}
+
+// The pages of a fresh host array appear at their first touch (about 0.25 µs
+// each): touched here, while the device still works, the values kept.
+static void touch_pages(void *p, size_t bytes) {
+    volatile uint8_t *b = static_cast<volatile uint8_t *>(p);
+    for (size_t off = 0; off < bytes; off += 4096) b[off] = b[off];
+}
+
+int pocr::download_staged(pocr_ctx *ctx, void *dst, const void *src, size_t bytes) {
+    RC(pin_halves(ctx));
+    const size_t piece = ctx->pin_half / 2;  // the copy out of one half overlaps the transfer into the other
+    const uint8_t *s8 = static_cast<const uint8_t *>(src);
+    uint8_t *d8 = static_cast<uint8_t *>(dst);
+    const size_t n = (bytes + piece - 1) / piece;
+    auto request = [&](size_t c) {
+        const size_t off = c * piece;
+        HIP_TRY(hipMemcpyAsync(ctx->pin + (c & 1) * ctx->pin_half, s8 + off, std::min(piece, bytes - off),
+                               hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(hipEventRecord(ctx->pin_ev[c & 1], ctx->stream));
+        return (int)POCR_OK;
+    };
+    for (size_t c = 0; c < std::min<size_t>(n, 2); ++c) RC(request(c));
+    touch_pages(dst, bytes);
+    for (size_t c = 0; c < n; ++c) {
+        const size_t off = c * piece;
+        HIP_TRY(hipEventSynchronize(ctx->pin_ev[c & 1]));
+        std::memcpy(d8 + off, ctx->pin + (c & 1) * ctx->pin_half, std::min(piece, bytes - off));
+        if (c + 2 < n) RC(request(c + 2));
+    }
+    return POCR_OK;
+}
+
+// Small parts: one kernel moves them between pinned host memory and their
+// places on the device (a copy call each costs the host 5-8 µs and a launch of
+// its own on the device).
+constexpr int kCopyParts = 4;
+constexpr size_t kSmallPart = 512u << 10;
+struct CopyParts {
+    const uint32_t *src[kCopyParts];
+    uint32_t *dst[kCopyParts];
+    int n[kCopyParts];
+};
+static __global__ void __launch_bounds__(kThreads) k_copy_parts(CopyParts p) {
+    const int y = blockIdx.y;
+    const uint32_t *src = y == 0 ? p.src[0] : (y == 1 ? p.src[1] : (y == 2 ? p.src[2] : p.src[3]));
+    uint32_t *dst = y == 0 ? p.dst[0] : (y == 1 ? p.dst[1] : (y == 2 ? p.dst[2] : p.dst[3]));
+    const int n = y == 0 ? p.n[0] : (y == 1 ? p.n[1] : (y == 2 ? p.n[2] : p.n[3]));
+    for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) dst[i] = src[i];
+}
+static int launch_copy_parts(pocr_ctx *ctx, const CopyParts &cp, int parts) {
+    int most = 0;
+    for (int i = 0; i < parts; ++i) most = std::max(most, cp.n[i]);
+    const int blocks = std::min(256, (most + kThreads - 1) / kThreads);
+    hipLaunchKernelGGL(k_copy_parts, dim3(blocks, parts), dim3(kThreads), 0, ctx->stream, cp);
+    HIP_TRY(hipGetLastError());
+    return POCR_OK;
+}
+static size_t pad256(size_t b) { return (b + 255) / 256 * 256; }
+static size_t small_bytes(std::initializer_list<HostPart> parts) {
+    size_t b = 0;
+    for (const HostPart &h : parts) b += h.bytes <= kSmallPart ? pad256(h.bytes) : 0;
+    return b;
+}
+
+int pocr::stage_in(pocr_ctx *ctx, std::initializer_list<HostPart> parts) {
+    CopyParts cp{};
+    int n = 0;
+    if (parts.size() > kCopyParts) return fail(POCR_ERR_ARG, "stage_in: %zu parts", parts.size());
+    const size_t need = small_bytes(parts);
+    if (ctx->in_used + need > ctx->small_in_n) {
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        ctx->in_used = 0;
+        RC(small_area(ctx, ctx->small_in, ctx->small_in_n, need));
+    }
+    for (const HostPart &h : parts) {
+        if (!h.bytes) continue;
+        if (h.bytes > kSmallPart) {
+            RC(upload_staged(ctx, h.dst, h.src, h.bytes));
+            continue;
+        }
+        uint8_t *pin = ctx->small_in + ctx->in_used;
+        std::memcpy(pin, h.src, h.bytes);
+        ctx->in_used += pad256(h.bytes);
+        cp.src[n] = reinterpret_cast<const uint32_t *>(pin);
+        cp.dst[n] = static_cast<uint32_t *>(h.dst);
+        cp.n[n++] = (int)(h.bytes / 4);
+    }
+    return n ? launch_copy_parts(ctx, cp, n) : POCR_OK;
+}
+
+int pocr::stage_out(pocr_ctx *ctx, std::initializer_list<HostPart> parts) {
+    CopyParts cp{};
+    int n = 0;
+    size_t off = 0;
+    if (parts.size() > kCopyParts) return fail(POCR_ERR_ARG, "stage_out: %zu parts", parts.size());
+    RC(small_area(ctx, ctx->small_out, ctx->small_out_n, small_bytes(parts)));
+    for (const HostPart &h : parts) {
+        if (!h.bytes || h.bytes > kSmallPart) continue;
+        cp.src[n] = static_cast<const uint32_t *>(h.src);
+        cp.dst[n] = reinterpret_cast<uint32_t *>(ctx->small_out + off);
+        cp.n[n++] = (int)(h.bytes / 4);
+        off += pad256(h.bytes);
+    }
+    if (n) RC(launch_copy_parts(ctx, cp, n));
+    for (const HostPart &h : parts) {
+        if (h.bytes > kSmallPart) RC(download_staged(ctx, h.dst, h.src, h.bytes));
+        else if (h.bytes) touch_pages(h.dst, h.bytes);
+    }
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    ctx->in_used = 0;
+    off = 0;
+    for (const HostPart &h : parts) {
+        if (!h.bytes || h.bytes > kSmallPart) continue;
+        std::memcpy(h.dst, ctx->small_out + off, h.bytes);
+        off += pad256(h.bytes);
     }
     return POCR_OK;
 }
@@ -767,10 +913,9 @@ extern "C" int pocr_matvec(pocr_ctx *ctx, const pocr_weight *w, const float *x, 
     hipStream_t s = ctx->stream;
     RC(ctx->x.ensure((size_t)m * w->cols * 4));
     RC(ctx->out.ensure((size_t)m * w->rows * 4));
-    RC(h2d(s, ctx->x.p, x, (size_t)m * w->cols * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)m * w->cols * 4}}));
     RC(matvec_rows(ctx, w, ctx->x.as<float>(), m, ctx->out.as<float>()));
-    RC(d2h(s, out, ctx->out.p, (size_t)m * w->rows * 4));
-    return sync(s);
+    return stage_out(ctx, {{out, ctx->out.p, (size_t)m * w->rows * 4}});
 }
 
 // m rows of x against one weight in the VNNI activation mode (Q8: plain)
@@ -782,15 +927,14 @@ extern "C" int pocr_matvec_vnni(pocr_ctx *ctx, const pocr_weight *w, const float
     hipStream_t s = ctx->stream;
     RC(ctx->x.ensure((size_t)m * w->cols * 4));
     RC(ctx->out.ensure((size_t)m * w->rows * 4));
-    RC(h2d(s, ctx->x.p, x, (size_t)m * w->cols * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)m * w->cols * 4}}));
     for (int r = 0; r < m; ++r) {
         GemvParams p = gemv_params_1(w);
         p.x = ctx->x.as<float>() + (size_t)r * w->cols;
         p.out = ctx->out.as<float>() + (size_t)r * w->rows;
         RC(gemv_launch_vnni(s, p, 1, PRO_COPY, EPI_PLAIN, kBigGrid));
     }
-    RC(d2h(s, out, ctx->out.p, (size_t)m * w->rows * 4));
-    return sync(s);
+    return stage_out(ctx, {{out, ctx->out.p, (size_t)m * w->rows * 4}});
 }
 
 // greedy argmax key of a step state: the max over the LM head's slots
@@ -816,15 +960,14 @@ extern "C" int pocr_matvec_argmax(pocr_ctx *ctx, const pocr_weight *w, const flo
     hipStream_t s = ctx->stream;
     RC(ctx->x.ensure((size_t)w->cols * 4));
     RC(ctx->state.ensure(sizeof(StepState)));
-    RC(h2d(s, ctx->x.p, x, (size_t)w->cols * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)w->cols * 4}}));
     HIP_TRY(hipMemsetAsync(ctx->state.p, 0, sizeof(StepState), s));
     GemvParams p = gemv_params_1(w);
     p.x = ctx->x.as<float>();
     p.st = ctx->state.as<StepState>();
     RC(gemv_launch(s, p, 1, PRO_COPY, EPI_ARGMAX, kBigGrid));
     StepState hst;
-    RC(d2h(s, &hst, ctx->state.p, sizeof(StepState)));
-    RC(sync(s));
+    RC(stage_out(ctx, {{&hst, ctx->state.p, sizeof(StepState)}}));
     if (hst.err) return fail(POCR_ERR_DEVICE, "matvec_argmax: device error %d", hst.err);
     const unsigned long long key = argmax_of(hst);
     if (key == 0ull) return fail(POCR_ERR_DEVICE, "matvec_argmax: no finite score");
@@ -1034,11 +1177,10 @@ static int ctx_topk(pocr_ctx *ctx, int rows, int k, int sample, const SampleStat
     hipStream_t s = ctx->stream;
     RC(ctx->topk_part.ensure((size_t)kTopKMaxParts * kTopKMax * 8));
     RC(ctx->samp.ensure(sizeof(SampleState)));
-    RC(h2d(s, ctx->samp.p, &in, sizeof(SampleState)));
+    RC(stage_in(ctx, {{ctx->samp.p, &in, sizeof(SampleState)}}));
     RC(enqueue_topk(s, ctx->out.as<float>(), rows, k, ctx->topk_part.as<unsigned long long>(),
                     ctx->samp.as<SampleState>(), nullptr, sample));
-    RC(d2h(s, out, ctx->samp.p, sizeof(SampleState)));
-    return sync(s);
+    return stage_out(ctx, {{out, ctx->samp.p, sizeof(SampleState)}});
 }
 
 extern "C" int pocr_matvec_topk(pocr_ctx *ctx, const pocr_weight *w, const float *x, int k, int32_t *ids,
@@ -1050,7 +1192,7 @@ extern "C" int pocr_matvec_topk(pocr_ctx *ctx, const pocr_weight *w, const float
     hipStream_t s = ctx->stream;
     RC(ctx->x.ensure((size_t)w->cols * 4));
     RC(ctx->out.ensure((size_t)w->rows * 4));
-    RC(h2d(s, ctx->x.p, x, (size_t)w->cols * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)w->cols * 4}}));
     GemvParams p = gemv_params_1(w);
     p.x = ctx->x.as<float>();
     p.out = ctx->out.as<float>();
@@ -1060,8 +1202,7 @@ extern "C" int pocr_matvec_topk(pocr_ctx *ctx, const pocr_weight *w, const float
         RC(wide_bufs(ctx->wide, w->rows, &b));
         RC(enqueue_sample_sorted(s, ctx->out.as<float>(), w->rows, k, b, nullptr, nullptr, 0));
         std::vector<unsigned long long> keys((size_t)k);
-        RC(d2h(s, keys.data(), b.keys, (size_t)k * 8));
-        RC(sync(s));
+        RC(stage_out(ctx, {{keys.data(), b.keys, (size_t)k * 8}}));
         keys_to_host(keys, k, ids, scores);
         return k;
     }
@@ -1083,7 +1224,7 @@ extern "C" int pocr_sample_topk(pocr_ctx *ctx, const float *logits, int n, int k
     CTX_GUARD(ctx);
     hipStream_t s = ctx->stream;
     RC(ctx->out.ensure((size_t)n * 4));
-    RC(h2d(s, ctx->out.p, logits, (size_t)n * 4));
+    RC(stage_in(ctx, {{ctx->out.p, logits, (size_t)n * 4}}));
     SampleState in{}, out;
     in.rng = *rng_state;
     in.temperature = temperature;
@@ -1092,7 +1233,7 @@ extern "C" int pocr_sample_topk(pocr_ctx *ctx, const float *logits, int n, int k
         WideBufs b;
         RC(wide_bufs(ctx->wide, n, &b));
         RC(ctx->samp.ensure(sizeof(SampleState)));
-        RC(h2d(s, ctx->samp.p, &in, sizeof(SampleState)));
+        RC(stage_in(ctx, {{ctx->samp.p, &in, sizeof(SampleState)}}));
         HIP_TRY(hipMemsetAsync(b.checks, 0, 4 * 4, s));
         RC(enqueue_sample_sorted(s, ctx->out.as<float>(), n, k, b, ctx->samp.as<SampleState>(), nullptr, 1));
         std::vector<unsigned long long> keys((size_t)k);
@@ -1123,14 +1264,14 @@ extern "C" int pocr_sample_full(pocr_ctx *ctx, const float *logits, int n, doubl
     CTX_GUARD(ctx);
     hipStream_t s = ctx->stream;
     RC(ctx->out.ensure((size_t)n * 4));
-    RC(h2d(s, ctx->out.p, logits, (size_t)n * 4));
+    RC(stage_in(ctx, {{ctx->out.p, logits, (size_t)n * 4}}));
     SampleState in{}, out;
     in.rng = *rng_state;
     in.temperature = temperature;
     WideBufs b;
     RC(wide_bufs(ctx->wide, n, &b));
     RC(ctx->samp.ensure(sizeof(SampleState)));
-    RC(h2d(s, ctx->samp.p, &in, sizeof(SampleState)));
+    RC(stage_in(ctx, {{ctx->samp.p, &in, sizeof(SampleState)}}));
     HIP_TRY(hipMemsetAsync(b.checks, 0, 4 * 4, s));
     RC(enqueue_sample_full(s, ctx->out.as<float>(), n, b, ctx->samp.as<SampleState>(), nullptr));
     RC(d2h(s, &out, ctx->samp.p, sizeof(SampleState)));
@@ -1146,7 +1287,7 @@ static int fused3(pocr_ctx *ctx, const pocr_weight *a, const pocr_weight *b, con
     const int rows = a->rows + b->rows + c->rows;
     RC(ctx->x.ensure((size_t)a->cols * 4));
     RC(ctx->out.ensure((size_t)rows * 4));
-    RC(h2d(s, ctx->x.p, x, (size_t)a->cols * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)a->cols * 4}}));
     GemvParams p{};
     p.m[0] = dev_mat(a);
     p.m[1] = dev_mat(b);
@@ -1178,10 +1319,9 @@ extern "C" int pocr_fused_matvec3(pocr_ctx *ctx, const pocr_weight *a, const poc
     hipStream_t s = ctx->stream;
     RC(fused3(ctx, a, b, c, x));
     float *o = ctx->out.as<float>();
-    RC(d2h(s, out_a, o, (size_t)a->rows * 4));
-    RC(d2h(s, out_b, o + a->rows, (size_t)b->rows * 4));
-    RC(d2h(s, out_c, o + a->rows + b->rows, (size_t)c->rows * 4));
-    return sync(s);
+    return stage_out(ctx, {{out_a, o, (size_t)a->rows * 4},
+                           {out_b, o + a->rows, (size_t)b->rows * 4},
+                           {out_c, o + a->rows + b->rows, (size_t)c->rows * 4}});
 }
 
 extern "C" int pocr_fused_matvec3_mrope(pocr_ctx *ctx, const pocr_weight *a, const pocr_weight *b,
@@ -1199,17 +1339,16 @@ extern "C" int pocr_fused_matvec3_mrope(pocr_ctx *ctx, const pocr_weight *a, con
     RC(fused3(ctx, a, b, c, x));
     const int half = head_dim / 2;
     RC(ctx->tabs.ensure((size_t)half * 8));
-    RC(h2d(s, ctx->tabs.p, cos_t, (size_t)half * 4));
-    RC(h2d(s, ctx->tabs.as<float>() + half, sin_t, (size_t)half * 4));
+    RC(stage_in(ctx, {{ctx->tabs.p, cos_t, (size_t)half * 4},
+                      {ctx->tabs.as<float>() + half, sin_t, (size_t)half * 4}}));
     float *o = ctx->out.as<float>();
     const int total = (q_heads + kv_heads) * half;
     hipLaunchKernelGGL(k_rope, dim3((total + kThreads - 1) / kThreads), dim3(kThreads), 0, s, o, o + a->rows,
                        ctx->tabs.as<float>(), ctx->tabs.as<float>() + half, q_heads, kv_heads, head_dim);
     HIP_TRY(hipGetLastError());
-    RC(d2h(s, out_a, o, (size_t)a->rows * 4));
-    RC(d2h(s, out_b, o + a->rows, (size_t)b->rows * 4));
-    RC(d2h(s, out_c, o + a->rows + b->rows, (size_t)c->rows * 4));
-    return sync(s);
+    return stage_out(ctx, {{out_a, o, (size_t)a->rows * 4},
+                           {out_b, o + a->rows, (size_t)b->rows * 4},
+                           {out_c, o + a->rows + b->rows, (size_t)c->rows * 4}});
 }
 
 extern "C" int pocr_swiglu_gate_up(pocr_ctx *ctx, const pocr_weight *gate, const pocr_weight *up, const float *x,
@@ -1222,27 +1361,27 @@ extern "C" int pocr_swiglu_gate_up(pocr_ctx *ctx, const pocr_weight *gate, const
     hipStream_t s = ctx->stream;
     RC(ctx->x.ensure((size_t)gate->cols * 4));
     RC(ctx->out.ensure((size_t)gate->rows * 4));
-    RC(h2d(s, ctx->x.p, x, (size_t)gate->cols * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)gate->cols * 4}}));
     GemvParams p = gemv_params_1(gate);
     p.m[1] = dev_mat(up);
     p.x = ctx->x.as<float>();
     p.out = ctx->out.as<float>();
     RC(gemv_launch(s, p, 2, PRO_COPY, EPI_SWIGLU, kBigGrid));
-    RC(d2h(s, out, ctx->out.p, (size_t)gate->rows * 4));
-    return sync(s);
+    return stage_out(ctx, {{out, ctx->out.p, (size_t)gate->rows * 4}});
 }
 
 // v = residual + W·x_dev (x already on the device), norm_out = RMSNorm(v)·norm_w,
 // residual = v iff in_place; host residual/norm_w/norm_out, synchronous
+// (staged: residual and norm_w are in ctx->res already)
 static int matvec_add_rmsnorm_dev(pocr_ctx *ctx, const pocr_weight *w, const float *x_dev, float *residual,
-                                  const float *norm_w, float eps, int in_place, float *norm_out) {
+                                  const float *norm_w, float eps, int in_place, float *norm_out, bool staged = false) {
     hipStream_t s = ctx->stream;
     const int n = w->rows;
     RC(ctx->res.ensure((size_t)n * 4 * 2));
     RC(ctx->vbuf.ensure((size_t)n * 4));
     RC(ctx->out3.ensure((size_t)n * 4));
-    RC(h2d(s, ctx->res.p, residual, (size_t)n * 4));
-    RC(h2d(s, ctx->res.as<float>() + n, norm_w, (size_t)n * 4));
+    if (!staged)
+        RC(stage_in(ctx, {{ctx->res.p, residual, (size_t)n * 4}, {ctx->res.as<float>() + n, norm_w, (size_t)n * 4}}));
     GemvParams p = gemv_params_1(w);
     p.x = x_dev;
     p.residual = ctx->res.as<float>();
@@ -1251,9 +1390,8 @@ static int matvec_add_rmsnorm_dev(pocr_ctx *ctx, const pocr_weight *w, const flo
     hipLaunchKernelGGL(k_rmsnorm, dim3(1), dim3(kThreads), 0, s, ctx->vbuf.as<float>(), ctx->res.as<float>() + n, n,
                        eps, ctx->out3.as<float>());
     HIP_TRY(hipGetLastError());
-    RC(d2h(s, norm_out, ctx->out3.p, (size_t)n * 4));
-    if (in_place) RC(d2h(s, residual, ctx->vbuf.p, (size_t)n * 4));
-    return sync(s);
+    return stage_out(ctx, {{norm_out, ctx->out3.p, (size_t)n * 4},
+                           {residual, ctx->vbuf.p, in_place ? (size_t)n * 4 : 0}});
 }
 
 extern "C" int pocr_matvec_add_rmsnorm(pocr_ctx *ctx, const pocr_weight *w, const float *x, float *residual,
@@ -1263,16 +1401,21 @@ extern "C" int pocr_matvec_add_rmsnorm(pocr_ctx *ctx, const pocr_weight *w, cons
     CHECK_INJECT("matvec_add_rmsnorm");
     CTX_GUARD(ctx);
     RC(ctx->x.ensure((size_t)w->cols * 4));
-    RC(h2d(ctx->stream, ctx->x.p, x, (size_t)w->cols * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)w->cols * 4}}));
     return matvec_add_rmsnorm_dev(ctx, w, ctx->x.as<float>(), residual, norm_w, eps, in_place, norm_out);
 }
 
 // SiLU(G·x)·(U·x) of host x into ctx->out (device), for the SwiGLU-down ops
-static int swiglu_dev(pocr_ctx *ctx, const pocr_weight *gate, const pocr_weight *up, const float *x) {
+// and, staged along with x, two host arrays of n floats into ctx->res
+static int swiglu_dev(pocr_ctx *ctx, const pocr_weight *gate, const pocr_weight *up, const float *x,
+                      const float *res = nullptr, const float *norm_w = nullptr, int n = 0) {
     hipStream_t s = ctx->stream;
     RC(ctx->x.ensure((size_t)gate->cols * 4));
     RC(ctx->out.ensure((size_t)gate->rows * 4));
-    RC(h2d(s, ctx->x.p, x, (size_t)gate->cols * 4));
+    if (n) RC(ctx->res.ensure((size_t)n * 4 * 2));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)gate->cols * 4},
+                      {ctx->res.p, res, (size_t)n * 4},
+                      {ctx->res.as<float>() + n, norm_w, (size_t)n * 4}}));
     GemvParams p = gemv_params_1(gate);
     p.m[1] = dev_mat(up);
     p.x = ctx->x.as<float>();
@@ -1301,8 +1444,7 @@ extern "C" int pocr_swiglu_down(pocr_ctx *ctx, const pocr_weight *gate, const po
     p.x = ctx->out.as<float>();
     p.out = ctx->out2.as<float>();
     RC(gemv_launch(s, p, 1, PRO_COPY, EPI_PLAIN, kBigGrid));
-    RC(d2h(s, out, ctx->out2.p, (size_t)down->rows * 4));
-    return sync(s);
+    return stage_out(ctx, {{out, ctx->out2.p, (size_t)down->rows * 4}});
 }
 
 extern "C" int pocr_swiglu_down_add_rmsnorm(pocr_ctx *ctx, const pocr_weight *gate, const pocr_weight *up,
@@ -1313,8 +1455,8 @@ extern "C" int pocr_swiglu_down_add_rmsnorm(pocr_ctx *ctx, const pocr_weight *ga
     RC(swiglu_down_args(gate, up, down, "pocr_swiglu_down_add_rmsnorm"));
     CHECK_INJECT("swiglu_down_add_rmsnorm");
     CTX_GUARD(ctx);
-    RC(swiglu_dev(ctx, gate, up, x));
-    return matvec_add_rmsnorm_dev(ctx, down, ctx->out.as<float>(), residual, norm_w, eps, in_place, norm_out);
+    RC(swiglu_dev(ctx, gate, up, x, residual, norm_w, down->rows));
+    return matvec_add_rmsnorm_dev(ctx, down, ctx->out.as<float>(), residual, norm_w, eps, in_place, norm_out, true);
 }
 
 extern "C" int pocr_add_rmsnorm(pocr_ctx *ctx, float *dst, const float *add, const float *w, int n, float eps,
@@ -1327,15 +1469,11 @@ extern "C" int pocr_add_rmsnorm(pocr_ctx *ctx, float *dst, const float *add, con
     RC(ctx->vbuf.ensure((size_t)n * 4));
     RC(ctx->out.ensure((size_t)n * 4));
     float *xd = ctx->x.as<float>();
-    RC(h2d(s, xd, dst, (size_t)n * 4));
-    RC(h2d(s, xd + n, add, (size_t)n * 4));
-    RC(h2d(s, xd + 2 * n, w, (size_t)n * 4));
+    RC(stage_in(ctx, {{xd, dst, (size_t)n * 4}, {xd + n, add, (size_t)n * 4}, {xd + 2 * n, w, (size_t)n * 4}}));
     hipLaunchKernelGGL(k_add_rmsnorm, dim3(1), dim3(kThreads), 0, s, xd, xd + n, xd + 2 * n, n, eps,
                        ctx->vbuf.as<float>(), ctx->out.as<float>());
     HIP_TRY(hipGetLastError());
-    RC(d2h(s, out, ctx->out.p, (size_t)n * 4));
-    if (in_place) RC(d2h(s, dst, ctx->vbuf.p, (size_t)n * 4));
-    return sync(s);
+    return stage_out(ctx, {{out, ctx->out.p, (size_t)n * 4}, {dst, ctx->vbuf.p, in_place ? (size_t)n * 4 : 0}});
 }
 
 extern "C" int pocr_mrope(pocr_ctx *ctx, float *x, const float *cos_t, const float *sin_t, int heads, int head_dim) {
@@ -1348,15 +1486,14 @@ extern "C" int pocr_mrope(pocr_ctx *ctx, float *x, const float *cos_t, const flo
     const size_t nx = (size_t)heads * head_dim;
     RC(ctx->x.ensure(nx * 4));
     RC(ctx->tabs.ensure((size_t)half * 8));
-    RC(h2d(s, ctx->x.p, x, nx * 4));
-    RC(h2d(s, ctx->tabs.p, cos_t, (size_t)half * 4));
-    RC(h2d(s, ctx->tabs.as<float>() + half, sin_t, (size_t)half * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, nx * 4},
+                      {ctx->tabs.p, cos_t, (size_t)half * 4},
+                      {ctx->tabs.as<float>() + half, sin_t, (size_t)half * 4}}));
     const int total = heads * half;
     hipLaunchKernelGGL(k_rope, dim3((total + kThreads - 1) / kThreads), dim3(kThreads), 0, s, ctx->x.as<float>(),
                        ctx->x.as<float>(), ctx->tabs.as<float>(), ctx->tabs.as<float>() + half, heads, 0, head_dim);
     HIP_TRY(hipGetLastError());
-    RC(d2h(s, x, ctx->x.p, nx * 4));
-    return sync(s);
+    return stage_out(ctx, {{x, ctx->x.p, nx * 4}});
 }
 
 extern "C" int pocr_rmsnorm(pocr_ctx *ctx, const float *x, const float *w, int n, float eps, float *out) {
@@ -1366,13 +1503,11 @@ extern "C" int pocr_rmsnorm(pocr_ctx *ctx, const float *x, const float *w, int n
     hipStream_t s = ctx->stream;
     RC(ctx->x.ensure((size_t)n * 8));
     RC(ctx->out.ensure((size_t)n * 4));
-    RC(h2d(s, ctx->x.p, x, (size_t)n * 4));
-    RC(h2d(s, ctx->x.as<float>() + n, w, (size_t)n * 4));
+    RC(stage_in(ctx, {{ctx->x.p, x, (size_t)n * 4}, {ctx->x.as<float>() + n, w, (size_t)n * 4}}));
     hipLaunchKernelGGL(k_rmsnorm, dim3(1), dim3(kThreads), 0, s, ctx->x.as<float>(), ctx->x.as<float>() + n, n, eps,
                        ctx->out.as<float>());
     HIP_TRY(hipGetLastError());
-    RC(d2h(s, out, ctx->out.p, (size_t)n * 4));
-    return sync(s);
+    return stage_out(ctx, {{out, ctx->out.p, (size_t)n * 4}});
 }
 
 extern "C" int pocr_mrope_pair(pocr_ctx *ctx, float *q, float *k, const float *cos_t, const float *sin_t,
@@ -1386,18 +1521,16 @@ extern "C" int pocr_mrope_pair(pocr_ctx *ctx, float *q, float *k, const float *c
     const size_t nq = (size_t)q_heads * head_dim, nk = (size_t)kv_heads * head_dim;
     RC(ctx->x.ensure((nq + nk) * 4));
     RC(ctx->tabs.ensure((size_t)half * 8));
-    RC(h2d(s, ctx->x.p, q, nq * 4));
-    RC(h2d(s, ctx->x.as<float>() + nq, k, nk * 4));
-    RC(h2d(s, ctx->tabs.p, cos_t, (size_t)half * 4));
-    RC(h2d(s, ctx->tabs.as<float>() + half, sin_t, (size_t)half * 4));
+    RC(stage_in(ctx, {{ctx->x.p, q, nq * 4},
+                      {ctx->x.as<float>() + nq, k, nk * 4},
+                      {ctx->tabs.p, cos_t, (size_t)half * 4},
+                      {ctx->tabs.as<float>() + half, sin_t, (size_t)half * 4}}));
     const int total = (q_heads + kv_heads) * half;
     hipLaunchKernelGGL(k_rope, dim3((total + kThreads - 1) / kThreads), dim3(kThreads), 0, s, ctx->x.as<float>(),
                        ctx->x.as<float>() + nq, ctx->tabs.as<float>(), ctx->tabs.as<float>() + half, q_heads,
                        kv_heads, head_dim);
     HIP_TRY(hipGetLastError());
-    RC(d2h(s, q, ctx->x.p, nq * 4));
-    RC(d2h(s, k, ctx->x.as<float>() + nq, nk * 4));
-    return sync(s);
+    return stage_out(ctx, {{q, ctx->x.p, nq * 4}, {k, ctx->x.as<float>() + nq, nk * 4}});
 }
 
 // Rows per wave of the decode attention for a cache capacity: short caches
@@ -1444,9 +1577,9 @@ static int text_attention_dev(pocr_ctx *ctx, const float *q, const float *k_cach
     RC(ctx->kc.ensure(kvd * cache_len * 4));
     RC(ctx->vc.ensure(kvd * cache_len * 4));
     RC(ctx->out.ensure(nq * 4));
-    RC(h2d(s, ctx->x.p, q, nq * 4));
-    RC(h2d(s, ctx->kc.p, k_cache, kvd * cache_len * 4));
-    RC(h2d(s, ctx->vc.p, v_cache, kvd * cache_len * 4));
+    RC(stage_in(ctx, {{ctx->x.p, q, nq * 4},
+                      {ctx->kc.p, k_cache, kvd * cache_len * 4},
+                      {ctx->vc.p, v_cache, kvd * cache_len * 4}}));
     const float scale = (float)(1.0 / std::sqrt((double)head_dim));  // invSqrt, model.go:7391
     const int group = heads / kv_heads;
     if (head_dim == kHD && group <= kMaxGroup) {
@@ -1491,8 +1624,7 @@ extern "C" int pocr_text_attention(pocr_ctx *ctx, const float *q, const float *k
     CHECK_INJECT("text_attention");
     CTX_GUARD(ctx);
     RC(text_attention_dev(ctx, q, k_cache, v_cache, cache_len, heads, kv_heads, head_dim));
-    RC(d2h(ctx->stream, out, ctx->out.p, (size_t)heads * head_dim * 4));
-    return sync(ctx->stream);
+    return stage_out(ctx, {{out, ctx->out.p, (size_t)heads * head_dim * 4}});
 }
 
 static int attention_out_args(const pocr_weight *wo, int heads, int head_dim, const char *op) {
@@ -1517,8 +1649,7 @@ extern "C" int pocr_text_attention_out(pocr_ctx *ctx, const float *q, const floa
     p.x = ctx->out.as<float>();
     p.out = ctx->out2.as<float>();
     RC(gemv_launch(s, p, 1, PRO_COPY, EPI_PLAIN, kBigGrid));
-    RC(d2h(s, out, ctx->out2.p, (size_t)wo->rows * 4));
-    return sync(s);
+    return stage_out(ctx, {{out, ctx->out2.p, (size_t)wo->rows * 4}});
 }
 
 extern "C" int pocr_text_attention_out_add_rmsnorm(pocr_ctx *ctx, const float *q, const float *k_cache,
@@ -2513,22 +2644,18 @@ static int enqueue_step(pocr_seq *s, int mode, bool need_logits, bool want_logit
     return POCR_OK;
 }
 
-int pocr::read_state(pocr_seq *s, StepState *out) {
-    HIP_TRY(hipMemcpyAsync(out, s->st, sizeof(StepState), hipMemcpyDeviceToHost, s->m->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(s->m->ctx->stream));
-    return POCR_OK;
-}
+int pocr::read_state(pocr_seq *s, StepState *out) { return stage_out(s->m->ctx, {{out, s->st, sizeof(StepState)}}); }
 
 int pocr::step_locked(pocr_seq *s, const float *emb, const int32_t pos3[3], int need_logits, float *logits,
                        int32_t *token) {
     pocr_model *m = s->m;
     hipStream_t st = m->ctx->stream;
     if (s->len >= s->cap) return fail(POCR_ERR_ARG, "pocr_step: cache full (%d rows)", s->cap);
-    RC(h2d(st, s->h, emb, (size_t)m->cfg.hidden * 4));
-    RC(h2d(st, &s->st->pos, pos3, 12));
+    RC(stage_in(m->ctx, {{s->h, emb, (size_t)m->cfg.hidden * 4}, {&s->st->pos, pos3, 12}}));
     RC(enqueue_step(s, 0, need_logits != 0, logits != nullptr));
     StepState hs;
-    RC(read_state(s, &hs));
+    const bool out = need_logits && logits;
+    RC(stage_out(m->ctx, {{&hs, s->st, sizeof(StepState)}, {logits, s->logits, out ? (size_t)m->cfg.vocab * 4 : 0}}));
     if (hs.err) return fail(POCR_ERR_DEVICE, "step: device state error %d", hs.err);
     s->len = hs.len;
     if (need_logits) {
@@ -2536,9 +2663,6 @@ int pocr::step_locked(pocr_seq *s, const float *emb, const int32_t pos3[3], int 
             const unsigned long long key = argmax_of(hs);
             if (key == 0ull) return fail(POCR_ERR_DEVICE, "step: no finite logit");
             *token = (int32_t)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFull));
-        }
-        if (logits) {
-            HIP_TRY(hipMemcpy(logits, s->logits, (size_t)m->cfg.vocab * 4, hipMemcpyDeviceToHost));
         }
     }
     return POCR_OK;
@@ -2675,8 +2799,7 @@ static int decode_locked(pocr_seq *s, int32_t first_token, int32_t first_pos, in
     RC(set_state_eos(s, hs, eos, n_eos));
     for (int i = 0; i < kArgSlots; ++i) hs.argmax_slot[i * kSlotPitch] = 0ull;
     hs.argmax_slot[0] = (1ull << 32) | (unsigned long long)(0xFFFFFFFFu - (uint32_t)first_token);
-    HIP_TRY(hipMemcpyAsync(s->st, &hs, sizeof(hs), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));  // hs is reused as a read-back target below
+    RC(stage_in(ctx, {{s->st, &hs, sizeof(hs)}}));
     int produced = 0;  // tokens known on the host
     int launched = 0;
     s->device_tokens = 0;
@@ -3091,9 +3214,7 @@ int seed_first_token(pocr_seq *s, int32_t first_token, int32_t first_pos, const 
     RC(set_state_eos(s, hs, eos, n_eos));
     for (int k = 0; k < kArgSlots; ++k) hs.argmax_slot[k * kSlotPitch] = 0ull;
     hs.argmax_slot[0] = (1ull << 32) | (unsigned long long)(0xFFFFFFFFu - (uint32_t)first_token);
-    HIP_TRY(hipMemcpyAsync(s->st, &hs, sizeof(StepState), hipMemcpyHostToDevice, s->m->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(s->m->ctx->stream));
-    return POCR_OK;
+    return stage_in(s->m->ctx, {{s->st, &hs, sizeof(StepState)}});
 }
 
 int32_t pending_token(const StepState &hs) {

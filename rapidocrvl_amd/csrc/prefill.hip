@@ -395,8 +395,7 @@ int prefill_ids_locked(pocr_seq *s, const int32_t *ids, int n, const float *imag
         i = j;
     }
     // ids ride in the position buffer's tail (rows·3 int32 + n)
-    HIP_TRY(hipMemcpyAsync(b.pos + (size_t)3 * b.cap_rows, ids, (size_t)n * 4, hipMemcpyHostToDevice,
-                           m->ctx->stream));
+    RC(stage_in(m->ctx, {{b.pos + (size_t)3 * b.cap_rows, ids, (size_t)n * 4}}));
     hipLaunchKernelGGL(k_embed_rows, dim3(n), dim3(kThreads), 0, m->ctx->stream, b.pos + (size_t)3 * b.cap_rows, n,
                        image ? image_token : -1, m->embed, H, b.h);
     HIP_TRY(hipGetLastError());
@@ -414,7 +413,7 @@ int prefill_run(pocr_seq *s, int n, const int32_t *pos3, float *logits, int32_t 
     const int clen0 = s->len;
     const int npad = round_up(n, 32);
     PrefillBufs &b = s->pf;
-    HIP_TRY(hipMemcpyAsync(b.pos, pos3, (size_t)n * 12, hipMemcpyHostToDevice, st));
+    RC(stage_in(m->ctx, {{b.pos, pos3, (size_t)n * 12}}));
     const float eps = c.rms_norm_eps;
     const float scale = (float)(1.0 / std::sqrt((double)c.head_dim));
     const int qt = m->layers[0].w[POCR_W_Q]->qtype;
@@ -518,18 +517,16 @@ int prefill_run(pocr_seq *s, int n, const int32_t *pos3, float *logits, int32_t 
     hs.pos[0] = pos3[3 * (n - 1)];
     hs.pos[1] = pos3[3 * (n - 1) + 1];
     hs.pos[2] = pos3[3 * (n - 1) + 2];
-    HIP_TRY(hipMemcpyAsync(s->st, &hs, sizeof(hs), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));  // hs is a stack object
+    RC(stage_in(m->ctx, {{s->st, &hs, sizeof(hs)}}));
     RC(enqueue_lm_head(s, b.v + (size_t)(n - 1) * H, logits != nullptr));
     StepState out;
-    RC(read_state(s, &out));
+    RC(stage_out(m->ctx, {{&out, s->st, sizeof(out)}, {logits, s->logits, logits ? (size_t)c.vocab * 4 : 0}}));
     s->len = clen0 + n;
     if (token) {
         const unsigned long long key = argmax_of(out);
         if (key == 0ull) return fail(POCR_ERR_DEVICE, "prefill: no finite logit");
         *token = (int32_t)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFull));
     }
-    if (logits) HIP_TRY(hipMemcpy(logits, s->logits, (size_t)c.vocab * 4, hipMemcpyDeviceToHost));
     return POCR_OK;
 }
 

@@ -265,8 +265,7 @@ extern "C" int pocr_project_image(pocr_projector *p, const float *vision_rows, i
     int rows = 0;
     RC(project_upload_locked(p, vision_rows, grid_t, grid_h, grid_w, &dev, &rows));
     if (rows == 0) return 0;
-    HIP_TRY(hipMemcpyAsync(out, dev, (size_t)rows * p->td * 4, hipMemcpyDeviceToHost, p->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(p->ctx->stream));
+    RC(stage_out(p->ctx, {{out, dev, (size_t)rows * p->td * 4}}));
     return rows;
 }
 
