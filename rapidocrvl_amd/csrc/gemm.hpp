@@ -773,31 +773,37 @@ __device__ __forceinline__ int2 xcd_tile() {
 }
 
 // ---------------------------------------------------------------------------
-// Prefill GEMM with both operands streamed into LDS by direct loads
-// (global_load_lds: HBM → LDS with no staging registers) through a ring of
-// NST stages of 128 columns.  Workgroup: 4 waves along the rows × 32 tokens;
-// a wave owns RB blocks of 16 rows of each of its NMAT matrices (gate and up
-// side by side) × 32 tokens: NMAT·RB·2·3 MFMAs (row blocks × 2 token blocks ×
+// Prefill GEMM over stages of 128 columns: the digit planes of 32 tokens, shared
+// by the workgroup's 4 waves, stream into a two-slot LDS ring by direct loads
+// (global_load_lds: HBM → LDS with no staging registers); the weight codes, each
+// wave's own, go straight to registers, one stage ahead.  Waves lie along the
+// rows; a wave owns RB blocks of 16 rows of each of its NMAT matrices (gate and
+// up side by side) × 32 tokens: NMAT·RB·2·3 MFMAs (row blocks × 2 token blocks ×
 // 3 digit planes) per 64 columns.
 //
 // K order of the MFMA operands: in stage u, MFMA step s, lane group lg takes
 // columns 128u + 32lg + 16s .. +15 (A and B alike; inside a 16-column group
 // the digit planes follow the weight codes' own order).  So a lane's weight
-// bytes for a stage are contiguous (Q4 16 B, Q8 32 B, Q6 24 B of its row):
-// each lane loads exactly the A operand it will use, and the LDS ring only
-// decouples the loads from the MFMAs (no register cost for the prefetch).
-// The digit planes are shared by the 4 waves.
+// bytes for a stage are contiguous (Q4 16 B, Q8 32 B, Q6 24 B of its row), and
+// each lane loads exactly the A operand it will use.
 //
 // Both operands are read from HBM images in this load order (the digitizer's
-// tile layout, digit_off; the weight image, k_tile_weight), so each direct
-// load reads 64 lanes × 16 (or 12) consecutive bytes.  From the row-major
-// weights and [pl][n][K] planes a load touched 16 rows × 64 B, half of each
-// 128-byte line, and the loads took 2.5× as long.
+// tile layout, digit_off; the weight image, k_tile_weight), so each load reads
+// 64 lanes × 16 (or 12) consecutive bytes.  From the row-major weights and
+// [pl][n][K] planes a load touched 16 rows × 64 B, half of each 128-byte line,
+// and the loads took 2.5× as long.
 //
-// Per stage and wave: B 3 loads (1 KB each: 12 per workgroup), A NMAT·RB
-// (Q4) or 2·NMAT·RB (Q8, Q6) loads.  One barrier per stage: at its top every wave has waited
-// for its own loads of this stage, and every wave has finished the previous
-// stage, whose slot is then refilled NST−1 stages ahead.
+// Bound: LDS reads (each wave reads the stage's 12 KB of planes) and the MFMAs,
+// in about equal parts.  The weights used to pass through LDS too, which cost
+// most where their 12-byte (Q6) pieces met the banks: 2,403 tokens, Q6, µs,
+// through LDS → registers: gate/up 83.5 → 64.6, q|k|v 36.7 → 31.1, o_proj and
+// down (mean) 37.6 → 32.2; 1,345 tokens, Q4: 29.9 → 29.8, 15.9 → 15.7,
+// 18.0 → 17.2.
+//
+// Per stage and wave: B 3 loads (1 KB each: 12 per workgroup), A NMAT·RB (Q4) or
+// 2·NMAT·RB (Q8, Q6) loads.  One barrier per stage: at its top every wave has
+// waited for its own loads of this stage, and every wave has finished the
+// previous stage, whose slot then takes the next one.
 // ---------------------------------------------------------------------------
 constexpr int kStageCols = 128;
 
@@ -833,17 +839,9 @@ static __global__ void __launch_bounds__(kThreads) k_tile_weight(const uint8_t *
 #pragma unroll
     for (int w = 0; w < A::bytes / 4; ++w) dp[w] = sp[w];
 }
-// the direct load places lane i's bytes at 16·i for 12- and 16-byte loads alike
-constexpr int kLdsLaneStride = 16;
-
-template <int QT, int NMAT, int NST, int RB_, int NPL = 3>
-struct GemmLdsLayout {
-    static constexpr int RB = RB_;
-    static constexpr int b_bytes = 2 * NPL * 2 * 64 * 16;                                     // [s][pl][tb][lane]
-    static constexpr int a_wave = NMAT * RB * ALds<QT>::chunks * 64 * kLdsLaneStride;        // [mi][rb][c][lane]
-    static constexpr int stage = b_bytes + kWaves * a_wave;
-    static constexpr int total = NST * stage;
-};
+// LDS bytes of a stage: the digit planes of 32 tokens, [s][pl][tb][lane]
+template <int NPL>
+constexpr int kGemmStage = 2 * NPL * 2 * 64 * 16;
 
 // HBM → LDS load of BYTES (16 or 12) per lane: lane i's bytes land at
 // lds + 16·i.  Written as inline asm so the compiler's wait-count pass does
@@ -874,19 +872,15 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_barrier" ::: "memory");
 }
 
-template <int QT, int NMAT, int NST, int RB, int NPL = 3>
+template <int QT, int NMAT, int RB, int NPL = 3>
 static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int epi) {
-    static_assert(NST == 2 || NST == 3, "the main loop is unrolled over two or three slots");
     static_assert(NMAT * RB <= 4, "at most four row blocks per wave");
     static_assert(NPL == 3 || (NPL == 1 && QT != QT_Q8), "three digit planes, or one plane of VNNI bytes (Q4, Q6)");
-    using Lay = GemmLdsLayout<QT, NMAT, NST, RB, NPL>;
     constexpr int WR = 16 * RB;                 // rows per matrix and wave
     constexpr int TB = 2;
     constexpr int CH = ALds<QT>::chunks, AB = ALds<QT>::bytes;
-    constexpr int LPS = NPL + NMAT * RB * CH;   // loads per stage and wave
-    __shared__ __attribute__((aligned(16))) uint8_t slot0[Lay::stage];
-    __shared__ __attribute__((aligned(16))) uint8_t slot1[Lay::stage];
-    __shared__ __attribute__((aligned(16))) uint8_t slot2[NST == 3 ? Lay::stage : 16];
+    __shared__ __attribute__((aligned(16))) uint8_t slot0[kGemmStage<NPL>];
+    __shared__ __attribute__((aligned(16))) uint8_t slot1[kGemmStage<NPL>];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, lg = lane >> 4;
@@ -915,9 +909,13 @@ static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int 
         bsrc[i] = p.xd + ((size_t)tile.y * nst * 4 * NPL + j) * 1024 + lane * 16;
         boff[i] = j * 1024;
     }
-    const int aoff = Lay::b_bytes + wave * Lay::a_wave;
 
-    auto issue = [&](int u, uint8_t *st) {
+    // a stage's weight bytes of this lane (the wave's own: straight to registers)
+    struct Raw {
+        uint32_t d[NMAT][RB][ALds<QT>::lane_words];
+    };
+    Raw raw0, raw1;
+    auto issue = [&](int u, uint8_t *st, Raw &raw) {
 #pragma unroll
         for (int i = 0; i < NPL; ++i) lds_load<16>(bsrc[i] + (size_t)4 * NPL * 1024 * u, st + boff[i]);
 #pragma unroll
@@ -925,9 +923,18 @@ static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int 
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                for (int c = 0; c < CH; ++c)
-                    lds_load<AB>(asrc[mi][rb] + (size_t)BS * u + c * 64 * AB,
-                                 st + aoff + ((mi * RB + rb) * CH + c) * 64 * kLdsLaneStride);
+                for (int c = 0; c < CH; ++c) {
+                    const uint8_t *q = asrc[mi][rb] + (size_t)BS * u + c * 64 * AB;
+                    uint32_t *d = raw.d[mi][rb];
+                    if constexpr (AB == 16) {
+                        const uint4 v = *reinterpret_cast<const uint4 *>(q);
+                        d[4 * c] = v.x; d[4 * c + 1] = v.y; d[4 * c + 2] = v.z; d[4 * c + 3] = v.w;
+                    } else {
+                        const uint3 v = *reinterpret_cast<const uint3 *>(q);
+                        d[3 * c] = v.x; d[3 * c + 1] = v.y; d[3 * c + 2] = v.z;
+                    }
+                }
+        __builtin_amdgcn_sched_barrier(0);  // all requested before the stage's MFMAs
     };
 
     v4i acc[NMAT][RB][TB][NPL];
@@ -940,25 +947,8 @@ static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int 
 #pragma unroll
                 for (int pl = 0; pl < NPL; ++pl) acc[mi][rb][tb][pl] = v4i{0, 0, 0, 0};
 
-    auto compute = [&](const uint8_t *st) {
+    auto compute = [&](const uint8_t *st, const Raw &raw) {
         const v4i *bl = reinterpret_cast<const v4i *>(st);
-        uint32_t raw[NMAT][RB][ALds<QT>::lane_words];  // the stage's weight bytes of this lane
-#pragma unroll
-        for (int mi = 0; mi < NMAT; ++mi)
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                for (int c = 0; c < CH; ++c) {
-                    const uint8_t *q = st + aoff + (((mi * RB + rb) * CH + c) * 64 + lane) * kLdsLaneStride;
-                    if constexpr (AB == 16) {
-                        const uint4 v = *reinterpret_cast<const uint4 *>(q);
-                        raw[mi][rb][4 * c] = v.x; raw[mi][rb][4 * c + 1] = v.y;
-                        raw[mi][rb][4 * c + 2] = v.z; raw[mi][rb][4 * c + 3] = v.w;
-                    } else {
-                        const uint32_t *w = reinterpret_cast<const uint32_t *>(q);
-                        raw[mi][rb][3 * c] = w[0]; raw[mi][rb][3 * c + 1] = w[1]; raw[mi][rb][3 * c + 2] = w[2];
-                    }
-                }
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             v4i b[TB][NPL];
@@ -973,7 +963,7 @@ static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int 
                     RawCodes<QT> rcd;
                     constexpr int W = QT == QT_Q8 ? 4 : (QT == QT_Q4 ? 2 : 3);
 #pragma unroll
-                    for (int w = 0; w < W; ++w) rcd.d[w] = raw[mi][rb][W * s + w];
+                    for (int w = 0; w < W; ++w) rcd.d[w] = raw.d[mi][rb][W * s + w];
                     const v4i av = unpack_codes16<QT>(rcd);
 #pragma unroll
                     for (int tb = 0; tb < TB; ++tb)
@@ -984,40 +974,28 @@ static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int 
                 }
         }
     };
-    // stage u: wait for this wave's loads of u (stage u+1 may stay in flight),
-    // barrier (every wave's loads of u have landed; every wave is done with
-    // u−1, whose slot takes stage u+2), then the MFMAs of u
-    auto body = [&](int u, const uint8_t *cur, uint8_t *refill) {
-        if (u + 1 < nst) wait_vm<LPS>();
-        else wait_vm<0>();
+    // stage u: wait for this wave's loads of u, barrier (every wave's loads of
+    // u have landed; every wave is done with u−1, whose slot takes u+1), then
+    // the MFMAs of u while u+1 is in flight
+    auto body = [&](int u, const uint8_t *cur, Raw &raw, uint8_t *next, Raw &raw_next) {
+        wait_vm<0>();
+        // the compiler's own wait for the weight bytes belongs here: at their
+        // use it would count the direct loads of u+1, which it cannot see, and
+        // wait for those
+#pragma unroll
+        for (int mi = 0; mi < NMAT; ++mi)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int w = 0; w < ALds<QT>::lane_words; ++w) asm volatile("" : "+v"(raw.d[mi][rb][w]));
         lds_barrier();
-        if (u + 2 < nst) issue(u + 2, refill);
-        if (on) compute(cur);
+        if (u + 1 < nst) issue(u + 1, next, raw_next);
+        if (on) compute(cur, raw);
     };
-
-    if constexpr (NST == 3) {
-        issue(0, slot0);
-        if (nst > 1) issue(1, slot1);
-        for (int u = 0; u < nst; u += 3) {
-            body(u, slot0, slot2);
-            if (u + 1 < nst) body(u + 1, slot1, slot0);
-            if (u + 2 < nst) body(u + 2, slot2, slot1);
-        }
-    } else {
-        // two slots: stage u+1 is requested after the barrier of stage u
-        // (every wave is done with u−1, whose slot it takes) and lands while
-        // u is computed; the smaller ring lets two workgroups share a CU
-        auto body2 = [&](int u, const uint8_t *cur, uint8_t *next) {
-            wait_vm<0>();
-            lds_barrier();
-            if (u + 1 < nst) issue(u + 1, next);
-            if (on) compute(cur);
-        };
-        issue(0, slot0);
-        for (int u = 0; u < nst; u += 2) {
-            body2(u, slot0, slot1);
-            if (u + 1 < nst) body2(u + 1, slot1, slot0);
-        }
+    issue(0, slot0, raw0);
+    for (int u = 0; u < nst; u += 2) {
+        body(u, slot0, raw0, slot1, raw1);
+        if (u + 1 < nst) body(u + 1, slot1, raw1, slot0, raw0);
     }
     if (!on) return;
 

@@ -118,17 +118,17 @@ int launch_gemm_lds_rb(hipStream_t s, int qtype, const GemmParams &p, int epi, i
     const dim3 grid((p.rows + 64 * RB - 1) / (64 * RB), npad / 32);
     if (p.vnni) {  // one plane of VNNI bytes (Q4, Q6)
         switch (qtype) {
-        case QT_Q4: hipLaunchKernelGGL((k_gemm_lds<QT_Q4, NMAT, 2, RB, 1>), grid, dim3(kThreads), 0, s, p, epi); break;
-        case QT_Q6: hipLaunchKernelGGL((k_gemm_lds<QT_Q6, NMAT, 2, RB, 1>), grid, dim3(kThreads), 0, s, p, epi); break;
+        case QT_Q4: hipLaunchKernelGGL((k_gemm_lds<QT_Q4, NMAT, RB, 1>), grid, dim3(kThreads), 0, s, p, epi); break;
+        case QT_Q6: hipLaunchKernelGGL((k_gemm_lds<QT_Q6, NMAT, RB, 1>), grid, dim3(kThreads), 0, s, p, epi); break;
         default: return fail(POCR_ERR_UNSUPPORTED, "VNNI gemm: qtype %d", qtype);
         }
         HIP_TRY(hipGetLastError());
         return POCR_OK;
     }
     switch (qtype) {
-    case QT_Q8: hipLaunchKernelGGL((k_gemm_lds<QT_Q8, NMAT, 2, RB>), grid, dim3(kThreads), 0, s, p, epi); break;
-    case QT_Q4: hipLaunchKernelGGL((k_gemm_lds<QT_Q4, NMAT, 2, RB>), grid, dim3(kThreads), 0, s, p, epi); break;
-    case QT_Q6: hipLaunchKernelGGL((k_gemm_lds<QT_Q6, NMAT, 2, RB>), grid, dim3(kThreads), 0, s, p, epi); break;
+    case QT_Q8: hipLaunchKernelGGL((k_gemm_lds<QT_Q8, NMAT, RB>), grid, dim3(kThreads), 0, s, p, epi); break;
+    case QT_Q4: hipLaunchKernelGGL((k_gemm_lds<QT_Q4, NMAT, RB>), grid, dim3(kThreads), 0, s, p, epi); break;
+    case QT_Q6: hipLaunchKernelGGL((k_gemm_lds<QT_Q6, NMAT, RB>), grid, dim3(kThreads), 0, s, p, epi); break;
     default: return fail(POCR_ERR_UNSUPPORTED, "gemm: qtype %d", qtype);
     }
     HIP_TRY(hipGetLastError());
