@@ -872,6 +872,12 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_barrier" ::: "memory");
 }
 
+// this wave's LDS reads have returned (before a barrier after which other
+// waves' direct loads overwrite what it read)
+__device__ __forceinline__ void lds_reads_done() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
 template <int QT, int NMAT, int RB, int NPL = 3>
 static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int epi) {
     static_assert(NMAT * RB <= 4, "at most four row blocks per wave");
@@ -1169,12 +1175,21 @@ static __global__ void __launch_bounds__(kThreads) k_rope_append(float *qkv, int
 // with quad q of dim d at position q ^ ((d >> 1) & 7).  The XOR swizzles make
 // the attention kernel's operand reads bank-conflict free with unpadded rows.
 //
-// k_attn_prefill — workgroup: one KV head, 4 query heads of its group (one per
-// wave) and two 16-token tiles, i and NT−1−i, so every workgroup meets the
-// same number of key blocks under the causal mask.  Both tiles go in one pass
-// over the longer one's key blocks: each block image is loaded once for both
-// (HBM → LDS by direct loads, two slots of two blocks); per block and tile
-// each wave runs
+// k_attn_prefill — workgroup: one KV head, 2 query heads of its group × 2
+// parities of key blocks (a wave each) and a tile of 32 tokens in two halves of
+// 16, which share every operand read of a block.  Tiles differ in length under
+// the causal mask; the longest start first, and two workgroups share a CU (64 KB
+// of LDS each: K and V of one stage of two blocks, either refilled while the
+// other is used), so the chip stays full until the short ones run out.
+// Bound: LDS operand reads, MFMAs and the softmax's vector work, in about equal
+// parts, with two waves per SIMD to overlap them.
+//
+// k_attn_prefill_pair (below) splits the same work another way; results are the
+// same bits.  Measured per layer, 16 heads, µs, pair / this one, tokens: 64 13.1 /
+// 10.5, 256 17.4 / 16.0, 512 25.0 / 24.3, 768 32.9 / 33.8, 1,345 52.0 / 58.5,
+// 2,040 77.5 / 89.7, 2,100 (264 workgroups of the pair form: a second round)
+// 128.5 / 93.1, 2,500 156.1 / 112.9.
+// Per block and half each wave runs
 //   Sᵀ (keys × tokens) = K · Qᵀ     2 key tiles × 4 dim chunks × 3 MFMAs
 //   online softmax per token column (the column's keys sit in 4 lane groups)
 //   Oᵀ (dims × tokens) += Vᵀ · Pᵀ   8 dim tiles × 3 MFMAs, K index = keys
@@ -1276,15 +1291,269 @@ __device__ __forceinline__ float groups4_sum(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-constexpr int kPfThreads = 512;   // 8 waves: 4 query heads × 2 key-block parities
+constexpr int kPfThreads = 256;   // 4 waves: 2 query heads × 2 key-block parities
+constexpr int kPfTile = 2 * kPfTok;  // query tokens of a workgroup
 
-static __global__ void __launch_bounds__(kPfThreads) k_attn_prefill(const float *qkv, int stride, const uint8_t *img,
+// the pair form's workgroups for ntok tokens, and whether it is the faster one:
+// one workgroup per CU at most, from about 640 tokens of 16 heads on (the lines
+// lie where the two cross, measured above)
+inline int pf_pair_groups(int heads, int kvh, int ntok) {
+    const int tiles = (ntok + kPfTok - 1) / kPfTok;
+    return kvh * ((heads / kvh + 3) / 4) * ((tiles + 1) / 2);
+}
+inline bool pf_pair(int heads, int kvh, int ntok) {
+    const int n = pf_pair_groups(heads, kvh, ntok);
+    return n > 80 && n <= 256;
+}
+
+static __global__ void __launch_bounds__(kPfThreads, 2) k_attn_prefill(const float *qkv, int stride, const uint8_t *img,
+                                                               int nblk_img, int heads, int kvh, int ntok,
+                                                               int clen0, float scale, float *out, int out_stride) {
+    // one stage of two block images (blocks 2s, 2s+1), K and V apart: 64 KB
+    constexpr int kHalf = kPfImage / 2;  // bytes of a block's K (or V) planes
+    __shared__ __attribute__((aligned(16))) uint8_t kbuf[2 * kHalf];
+    __shared__ __attribute__((aligned(16))) uint8_t vbuf[2 * kHalf];
+    constexpr int LPB = 2 * kHalf / 1024 / (kPfThreads / 64);  // direct loads per buffer and wave (8)
+    const int group = heads / kvh;
+    const int pairs = (group + 1) / 2;
+    const int g = blockIdx.x / pairs, hp = blockIdx.x % pairs;
+    const int t = threadIdx.x, l = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int par = wave >> 1;                    // key-block parity of this wave
+    const int lr = l & 15, lg = l >> 4;
+    const int hl = 2 * hp + (wave & 1);           // head within the group
+    const bool wave_on = hl < group;              // uniform
+    const int hh = g * group + min(hl, group - 1);
+    const int tile = gridDim.y - 1 - blockIdx.y;  // longest first
+
+    // the tile's two halves of 16 tokens: both see every key block but the
+    // last one or two, whose operands are read from LDS once for both
+    int q0[2], my_last[2], nblk[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        q0[u] = tile * kPfTile + u * kPfTok;
+        my_last[u] = clen0 + min(q0[u] + lr, ntok - 1);  // this lane's token (clamped; stored only if < ntok)
+        nblk[u] = (clen0 + min(q0[u] + kPfTok, ntok) - 1) / kPfKeys + 1;
+    }
+    const int nblk_all = nblk[1];  // ≥ nblk[0]
+    const int nstage = (nblk_all + 1) / 2;
+
+    // K or V planes (which = 0, 1) of blocks 2s, 2s+1 (a missing 2s+1 repeats
+    // 2s, so every wave always has the same loads in flight); wave w takes the
+    // 1 KB pieces 8w.. of the 32
+    const uint8_t *gimg = img + (size_t)g * nblk_img * kPfImage + 16 * l;
+    auto issue = [&](int s, int which, uint8_t *buf) {
+        const int b0 = 2 * s, b1 = min(2 * s + 1, nblk_all - 1);
+#pragma unroll
+        for (int i = 0; i < LPB; ++i) {
+            const int piece = wave * LPB + i;
+            const int blk = piece < kHalf / 1024 ? b0 : b1;
+            lds_load<16>(gimg + (size_t)blk * kPfImage + which * kHalf + (piece & (kHalf / 1024 - 1)) * 1024,
+                         buf + piece * 1024);
+        }
+    };
+
+    // Qᵀ operands of the first product: token lr, dims 32c + 8lg + e
+    v8bf qh[2][4], ql[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const float *qs = qkv + (size_t)min(q0[u] + lr, ntok - 1) * stride + (size_t)hh * kHD + 8 * lg;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float4 a4 = *reinterpret_cast<const float4 *>(qs + 32 * c);
+            const float4 b4 = *reinterpret_cast<const float4 *>(qs + 32 * c + 4);
+            const float x[8] = {a4.x, a4.y, a4.z, a4.w, b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                __bf16 h, lo;
+                split_bf16(x[e], h, lo);
+                qh[u][c][e] = h;
+                ql[u][c][e] = lo;
+            }
+        }
+    }
+    v4f o[2][8];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) o[u][dt] = v4f{0.f, 0.f, 0.f, 0.f};
+    float m[2] = {-INFINITY, -INFINITY}, lsum[2] = {0.0f, 0.0f};
+    v4f sT[2][2];
+    v8bf ph[2], pl[2];
+
+    // Sᵀ of halves U0.. and 1 (U0 a compile-time 0 or 1) against block planes kb
+    auto scores = [&](const uint8_t *kb, auto first) {
+        constexpr int U0 = decltype(first)::value;
+        const __bf16 *im = reinterpret_cast<const __bf16 *>(kb);
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+            for (int u = U0; u < 2; ++u) sT[u][kt] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const v8bf kh = *reinterpret_cast<const v8bf *>(im + pf_k_at(0, 16 * kt + lr, 4 * c + lg));
+                const v8bf kl = *reinterpret_cast<const v8bf *>(im + pf_k_at(1, 16 * kt + lr, 4 * c + lg));
+#pragma unroll
+                for (int u = U0; u < 2; ++u)
+                    sT[u][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh[u][c], sT[u][kt], 0, 0, 0);
+#pragma unroll
+                for (int u = U0; u < 2; ++u)
+                    sT[u][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, ql[u][c], sT[u][kt], 0, 0, 0);
+#pragma unroll
+                for (int u = U0; u < 2; ++u)
+                    sT[u][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qh[u][c], sT[u][kt], 0, 0, 0);
+            }
+        }
+    };
+    // online softmax of half u's token column lr over block b (branch-free:
+    // masked keys get p = 0 by selection after an exp of a clamped argument)
+    auto softmax = [&](int b, int u) {
+        // scores are rounded (s·scale) before the max is subtracted
+#pragma clang fp contract(off)
+        const int k0 = b * kPfKeys;
+        float sv[8];
+        bool vis[8];
+        float mb = m[u];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                vis[4 * kt + i] = k0 + 16 * kt + 4 * lg + i <= my_last[u];
+                sv[4 * kt + i] = vis[4 * kt + i] ? sT[u][kt][i] * scale : -INFINITY;
+                mb = fmaxf(mb, sv[4 * kt + i]);
+            }
+        mb = groups4_max(mb);
+        // a column may have seen no visible key yet on this parity (mb = −∞):
+        // its p are all 0 and its running sums stay 0
+        const float mx = mb == -INFINITY ? 0.0f : mb;
+        float ps = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float ex = exp_hw(sv[e] - mx);
+            const float p = vis[e] ? ex : 0.0f;
+            ps += p;
+            __bf16 a, c;
+            split_bf16(p, a, c);
+            ph[u][e] = a;
+            pl[u][e] = c;
+        }
+        ps = groups4_sum(ps);
+        // rescale only when a column's maximum moved (exp_hw(0) is exactly
+        // 1, so skipping is exact)
+        if (__builtin_amdgcn_ballot_w64(mb != m[u])) {
+            const float fe = exp_hw(m[u] - mx);
+            const float f = m[u] == -INFINITY ? 0.0f : fe;
+            lsum[u] *= f;
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) o[u][dt] *= f;
+        }
+        lsum[u] += ps;
+        m[u] = mb;
+    };
+    // Oᵀ += Vᵀ·Pᵀ of halves U0.. and 1 against block planes vb
+    auto values = [&](const uint8_t *vb, auto first) {
+        constexpr int U0 = decltype(first)::value;
+        // pf_v_at counts from the block image's start, K planes first
+        const __bf16 *im = reinterpret_cast<const __bf16 *>(vb) - 2 * kPfKPlane;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) {
+            const int d = 16 * dt + lr;
+            const v4bf ah0 = *reinterpret_cast<const v4bf *>(im + pf_v_at(0, d, lg));
+            const v4bf ah1 = *reinterpret_cast<const v4bf *>(im + pf_v_at(0, d, 4 + lg));
+            const v4bf al0 = *reinterpret_cast<const v4bf *>(im + pf_v_at(1, d, lg));
+            const v4bf al1 = *reinterpret_cast<const v4bf *>(im + pf_v_at(1, d, 4 + lg));
+            const v8bf vh = __builtin_shufflevector(ah0, ah1, 0, 1, 2, 3, 4, 5, 6, 7);
+            const v8bf vl = __builtin_shufflevector(al0, al1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+            for (int u = U0; u < 2; ++u) o[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, ph[u], o[u][dt], 0, 0, 0);
+#pragma unroll
+            for (int u = U0; u < 2; ++u) o[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, pl[u], o[u][dt], 0, 0, 0);
+#pragma unroll
+            for (int u = U0; u < 2; ++u) o[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vl, ph[u], o[u][dt], 0, 0, 0);
+        }
+    };
+
+    // Stage s: this wave's block is 2s + parity.  Each buffer is refilled for
+    // s+1 as soon as every wave has read it, so K's loads run behind the
+    // softmax and P·V, V's behind the next scores; a wait leaves the other
+    // buffer's LPB loads in flight.
+    issue(0, 0, kbuf);
+    issue(0, 1, vbuf);
+    for (int s = 0; s < nstage; ++s) {
+        const bool more = s + 1 < nstage;
+        const int b = 2 * s + par;
+        const bool on1 = wave_on && b < nblk_all, on0 = on1 && b < nblk[0];  // uniform
+        wait_vm<LPB>();  // K(s); V(s) may be in flight
+        lds_barrier();
+        const uint8_t *kb = kbuf + par * kHalf, *vb = vbuf + par * kHalf;
+        if (on0) scores(kb, std::integral_constant<int, 0>{});
+        else if (on1) scores(kb, std::integral_constant<int, 1>{});
+        lds_reads_done();
+        lds_barrier();
+        if (more) issue(s + 1, 0, kbuf);
+        if (on0) softmax(b, 0);
+        if (on1) softmax(b, 1);
+        if (more) wait_vm<LPB>();  // V(s); K(s+1) may be in flight
+        else wait_vm<0>();
+        lds_barrier();
+        if (on0) values(vb, std::integral_constant<int, 0>{});
+        else if (on1) values(vb, std::integral_constant<int, 1>{});
+        lds_reads_done();
+        lds_barrier();
+        if (more) issue(s + 1, 1, vbuf);
+    }
+
+    // merge the two parities of each head through LDS, half 0 in kbuf, half 1
+    // in vbuf (free after the barrier: no loads are in flight)
+    if (par == 1) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            float *mrg = reinterpret_cast<float *>(u == 0 ? kbuf : vbuf) + (size_t)((wave & 1) * 64 + l) * 34;
+            mrg[0] = m[u];
+            mrg[1] = lsum[u];
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mrg[2 + 4 * dt + i] = o[u][dt][i];
+        }
+    }
+    __syncthreads();
+    if (par == 0 && wave_on) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (q0[u] + lr >= ntok) continue;
+            const float *mrg = reinterpret_cast<const float *>(u == 0 ? kbuf : vbuf) + (size_t)((wave & 1) * 64 + l) * 34;
+            const float m1 = mrg[0], l1 = mrg[1];
+            const float M = fmaxf(m[u], m1);  // finite: key 0 is in block 0
+            const float f0 = m[u] == -INFINITY ? 0.0f : exp_hw(m[u] - M);
+            const float f1 = m1 == -INFINITY ? 0.0f : exp_hw(m1 - M);
+            const float inv = 1.0f / (lsum[u] * f0 + l1 * f1);
+            float *dst = out + (size_t)(q0[u] + lr) * out_stride + (size_t)hh * kHD + 4 * lg;
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) {
+                float r[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r[i] = (o[u][dt][i] * f0 + mrg[2 + 4 * dt + i] * f1) * inv;
+                *reinterpret_cast<float4 *>(dst + 16 * dt) = make_float4(r[0], r[1], r[2], r[3]);
+            }
+        }
+    }
+}
+
+// The same attention by 4 query heads and two 16-token tiles, i and NT−1−i, per
+// workgroup: every workgroup meets the same number of key blocks under the
+// causal mask, both tiles in one pass over the longer one's blocks (two slots of
+// two blocks, 128 KB of LDS: one workgroup per CU).  Ahead while its grid is one
+// round of the chip and large: pf_pair.
+constexpr int kPfPairThreads = 512;   // 8 waves: 4 query heads × 2 key-block parities
+
+static __global__ void __launch_bounds__(kPfPairThreads) k_attn_prefill_pair(const float *qkv, int stride, const uint8_t *img,
                                                                int nblk_img, int heads, int kvh, int ntok,
                                                                int clen0, float scale, float *out, int out_stride) {
     // two stages of two block images (blocks 2s, 2s+1): 128 KB
     __shared__ __attribute__((aligned(16))) uint8_t stage0[2 * kPfImage];
     __shared__ __attribute__((aligned(16))) uint8_t stage1[2 * kPfImage];
-    constexpr int kW = kPfThreads / 64;
+    constexpr int kW = kPfPairThreads / 64;
     constexpr int LPS = 2 * kPfImage / 1024 / kW;  // direct loads per stage and wave (8)
     const int group = heads / kvh;
     const int quads = (group + 3) / 4;
@@ -1485,7 +1754,6 @@ static __global__ void __launch_bounds__(kPfThreads) k_attn_prefill(const float 
         }
     }
 }
-
 
 // Greedy choice over rows of logits (the batched LM head): workgroup (x, i)
 // scans its slice of row i and folds the best (score, index) key into argmax

@@ -474,12 +474,20 @@ int prefill_run(pocr_seq *s, int n, const int32_t *pos3, float *logits, int32_t 
             RC(launch_attn_ordered_rows(st, b.qkv, QKV, layer_k(s, li), layer_v(s, li), c.heads, c.kv_heads, n, clen0,
                                         scale, b.ho, Q));
         } else {
-            const int ntiles = (n + kPfTok - 1) / kPfTok, quads = (c.heads / c.kv_heads + 3) / 4;
             const int nblk = (clen0 + n + kPfKeys - 1) / kPfKeys;
             hipLaunchKernelGGL(k_kv_blocks, dim3(nblk, c.kv_heads), dim3(kThreads), 0, st, layer_k(s, li),
                                layer_v(s, li), c.kv_heads, clen0 + n, nblk, b.kvimg);
-            hipLaunchKernelGGL(k_attn_prefill, dim3(c.kv_heads * quads, (ntiles + 1) / 2), dim3(kPfThreads), 0, st,
-                               b.qkv, QKV, b.kvimg, nblk, c.heads, c.kv_heads, n, clen0, scale, b.ho, Q);
+            const int group = c.heads / c.kv_heads;
+            if (pf_pair(c.heads, c.kv_heads, n)) {
+                const int nt = (n + kPfTok - 1) / kPfTok;
+                hipLaunchKernelGGL(k_attn_prefill_pair, dim3(c.kv_heads * ((group + 3) / 4), (nt + 1) / 2),
+                                   dim3(kPfPairThreads), 0, st, b.qkv, QKV, b.kvimg, nblk, c.heads, c.kv_heads, n,
+                                   clen0, scale, b.ho, Q);
+            } else {
+                hipLaunchKernelGGL(k_attn_prefill, dim3(c.kv_heads * ((group + 1) / 2), (n + kPfTile - 1) / kPfTile),
+                                   dim3(kPfThreads), 0, st, b.qkv, QKV, b.kvimg, nblk, c.heads, c.kv_heads, n, clen0,
+                                   scale, b.ho, Q);
+            }
             HIP_TRY(hipGetLastError());
         }
         // 3. o_proj + residual (+ the Q4/Q6 behaviour per token) → v; h if in place

@@ -168,3 +168,36 @@ def test_prefill_gemm_layouts_agree(ctx, qtype, monkeypatch):
     for (a, b), (c, d) in zip(kvt, kvr):
         assert np.array_equal(a, c) and np.array_equal(b, d)
     gm.close()
+
+
+ODD = DecoderConfig(hidden=512, inter=1536, layers=2, heads=3, kv_heads=1, head_dim=128, vocab=1024, eps=1e-5,
+                    rope_theta=500000.0)
+
+
+@pytest.mark.parametrize("cfg,parts", [
+    (MID, (33,)), (MID, (17, 16)), (MID, (47, 18, 1)),       # halves and tiles that end inside a key block
+    (ODD, (65, 40)),                                         # a group of 3 heads: one wave idles
+    (MID, (320, 380)), (MID, (645, 60)),                     # a whole prompt on the pair form, parts on the other
+    (MID, (1040, 1040)),                                     # and the other way round
+], ids=str)
+def test_prefill_attention_forms_agree(ctx, cfg, parts):
+    """Both forms of the prompt attention take a token's key blocks in the same
+    order and parities, whatever tile it falls into: a prompt at once and in
+    parts gives the same bits."""
+    w = synth.make_weights(cfg, Q8, seed=41)
+    gm = lib.Model(ctx, cfg)
+    gm.load_weights(w)
+    n = sum(parts)
+    embs = w["embed"][synth.prompt_ids(n, seed=42, high=cfg.vocab)]
+    pos = np.array([[p, p, p] for p in range(n)], np.int32)
+    whole, split = gm.seq(n + 8), gm.seq(n + 8)
+    tok, lg = whole.prefill(embs, pos, want_logits=True)
+    at = 0
+    for m in parts:
+        tok2, lg2 = split.prefill(embs[at:at + m], pos[at:at + m], want_logits=True)
+        at += m
+    assert tok == tok2 and np.array_equal(lg, lg2)
+    for li in range(cfg.layers):
+        for a, b in zip(whole.read_kv(li), split.read_kv(li)):
+            assert np.array_equal(a, b)
+    gm.close()
