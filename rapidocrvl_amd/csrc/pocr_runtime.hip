@@ -2964,7 +2964,6 @@ GemmParams batch_gemm(const DecodeBatch &b, const pocr_weight *w, int K) {
     p.xs = b.xs;
     p.xb = b.xb;
     p.ntok = b.n;
-    p.rst = b.rst;
     return p;
 }
 
@@ -3182,7 +3181,7 @@ int enqueue_batch_step(DecodeBatch &b) {
         lp.ntok = b.ng;
         lp.out = b.logits;
         lp.out_stride = V;
-        RC(gemm_small_rows(st, m->lm->qtype, 1, lp, G_PLAIN));
+        RC(gemm_small_rows(st, m->lm->qtype, lp, G_PLAIN));
         constexpr int kSlice = 2048;
         hipLaunchKernelGGL(k_argmax_rows, dim3((V + kSlice - 1) / kSlice, b.ng), dim3(kThreads), 0, st, b.logits, V, V,
                            kSlice, b.rst);
