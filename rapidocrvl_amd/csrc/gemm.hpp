@@ -865,15 +865,12 @@ __device__ __forceinline__ void wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// workgroup barrier that keeps LDS reads and loads on their side of it
+// workgroup barrier that keeps LDS reads and loads on their side of it: this
+// wave's LDS reads have returned before it, since other waves' direct loads may
+// overwrite what it read right after.  (The compiler's own wait for a read
+// stands at the read's use, and the MFMAs may sink below a bare s_barrier.)
 __device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_barrier" ::: "memory");
-}
-
-// this wave's LDS reads have returned (before a barrier after which other
-// waves' direct loads overwrite what it read)
-__device__ __forceinline__ void lds_reads_done() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 template <int QT, int NMAT, int RB, int NPL = 3>
@@ -1486,7 +1483,6 @@ static __global__ void __launch_bounds__(kPfThreads, 2) k_attn_prefill(const flo
         const uint8_t *kb = kbuf + par * kHalf, *vb = vbuf + par * kHalf;
         if (on0) scores(kb, std::integral_constant<int, 0>{});
         else if (on1) scores(kb, std::integral_constant<int, 1>{});
-        lds_reads_done();
         lds_barrier();
         if (more) issue(s + 1, 0, kbuf);
         if (on0) softmax(b, 0);
@@ -1496,7 +1492,6 @@ static __global__ void __launch_bounds__(kPfThreads, 2) k_attn_prefill(const flo
         lds_barrier();
         if (on0) values(vb, std::integral_constant<int, 0>{});
         else if (on1) values(vb, std::integral_constant<int, 1>{});
-        lds_reads_done();
         lds_barrier();
         if (more) issue(s + 1, 1, vbuf);
     }
