@@ -3226,7 +3226,8 @@ int32_t pending_token(const StepState &hs) {
 int batch_alloc(DecodeBatch &b) {
     const pocr_config &c = b.m->cfg;
     const size_t H = c.hidden, Q = (size_t)c.heads * c.head_dim, KV = (size_t)c.kv_heads * c.head_dim;
-    const size_t rows = std::max(b.cap, b.nv);
+    // whole GEMV passes: the head's last pass over 3 sequences reads 4 rows
+    const size_t rows = (std::max(b.cap, b.nv) + kMaxNV - 1) / kMaxNV * kMaxNV;
     hipStream_t s = b.m->ctx->stream;
     for (auto pr : {std::make_pair(&b.h, H), std::make_pair(&b.v, H), std::make_pair(&b.qkv, Q + 2 * KV),
                     std::make_pair(&b.ho, Q), std::make_pair(&b.g, (size_t)c.intermediate)}) {
@@ -3236,7 +3237,7 @@ int batch_alloc(DecodeBatch &b) {
     }
     HIP_TRY(hipMalloc(&b.pad, sizeof(StepState)));
     HIP_TRY(hipMemsetAsync(b.pad, 0, sizeof(StepState), s));
-    if (rows >= (size_t)kBatchWideHeadMin) {
+    if (b.cap >= kBatchWideHeadMin) {
         const size_t kmax = std::max(std::max(H, Q), (size_t)c.intermediate);
         HIP_TRY(hipMalloc(&b.xd, 3 * 16 * kmax));
         HIP_TRY(hipMemsetAsync(b.xd, 0, 3 * 16 * kmax, s));
@@ -3245,7 +3246,7 @@ int batch_alloc(DecodeBatch &b) {
     }
     b.rows_ok[0] = batch_rows_ok(b.m, false);
     b.rows_ok[1] = batch_rows_ok(b.m, true);
-    if (b.rows_ok[0] || rows > (size_t)kMaxNV) HIP_TRY(hipMalloc(&b.rst, kMaxBatch * sizeof(StepState *)));
+    if (b.rows_ok[0] || b.cap > kMaxNV) HIP_TRY(hipMalloc(&b.rst, kMaxBatch * sizeof(StepState *)));
     if (b.rows_ok[0]) {
         // zeros: a row whose first step stops at once never writes its column
         const size_t img = rows_image_bytes((int)(H + Q) + c.intermediate), ssq = (H / 16) * 16 * sizeof(float);
@@ -3254,7 +3255,7 @@ int batch_alloc(DecodeBatch &b) {
         HIP_TRY(hipMalloc(&b.ssq, ssq));
         HIP_TRY(hipMemsetAsync(b.ssq, 0, ssq, s));
     }
-    if (rows > (size_t)kMaxNV) {
+    if (b.cap > kMaxNV) {
         if (gemm_small_ok(c.vocab, c.hidden)) HIP_TRY(hipMalloc(&b.logits, (size_t)16 * c.vocab * 4));
     }
     return POCR_OK;

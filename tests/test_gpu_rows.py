@@ -51,3 +51,23 @@ def test_rows_match_single_decode(ctx, cfg, qtype, nseq):
             for a, b in zip(batch[i].read_kv(li), s.read_kv(li)):
                 err = np.linalg.norm(a - b) / np.linalg.norm(b)
                 assert err < 2e-5, (i, li, err)
+
+
+@pytest.mark.parametrize("nseq", [7, 11])
+def test_head_pass_over_the_last_three_rows(ctx, nseq):
+    # 512 columns and 1,000 rows: the greedy head runs 4-vector passes, the last
+    # one over three sequences and a padding row past them
+    cfg = DecoderConfig(hidden=512, inter=1536, layers=1, heads=4, kv_heads=1, head_dim=128, vocab=1000, eps=1e-5,
+                        rope_theta=500000.0)
+    m = lib.Model(ctx, cfg)
+    m.load_weights(synth.make_weights(cfg, Q8, seed=33))
+    prompts = [synth.prompt_ids(3 + i, seed=500 + i, high=cfg.vocab) for i in range(nseq)]
+    seqs, want = [], []
+    for ids in prompts:
+        s = m.seq(len(ids) + 12)
+        first = int(s.generate(ids, 1, eos=(), use_prefill=True)[0])
+        want.append(list(s.decode_greedy(first, len(ids), 8, eos=())))
+        s.truncate(len(ids))
+        seqs.append((s, first))
+    got = lib.decode_batch([s for s, _ in seqs], [f for _, f in seqs], [len(ids) for ids in prompts], 8, eos=())
+    assert [list(g) for g in got] == want
