@@ -2855,12 +2855,12 @@ extern "C" int pocr_decode_greedy(pocr_seq *s, int32_t first_token, int32_t firs
 }
 
 // ---------------------------------------------------------------------------
-// Batched greedy decode: up to kMaxBatch sequences of one model advance together.
-// Every layer GEMV streams its weights once for all of them (NV activation
-// vectors per pass, padded to 2 or 4), attention and its merge run in one
-// launch each with the sequence in blockIdx.z, and each sequence keeps its own
-// KV cache, step state and token buffer.  One step is captured into a HIP
-// graph and replayed; the host reads the states back every 16 steps.
+// Batched decode: up to kMaxBatch sequences of one model advance together.
+// Every layer matrix is read once for all of them (batch_layer_rows), attention
+// and its merge run in one launch each with the sequence in blockIdx.z, and each
+// sequence keeps its own KV cache, step state and token buffer.  One step is
+// captured into a HIP graph and replayed; the host reads the states back every
+// 16 steps.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -2872,8 +2872,7 @@ struct DecodeBatch {
     pocr_model *m = nullptr;
     int n = 0;    // sequences: the ng greedy ones first, then the sampling ones
     int ng = 0;
-    int nv = 1;   // vectors per GEMV pass (n ≤ 4: n padded to 1, 2 or 4)
-    int cap = 0;  // vector rows the buffers hold (≥ nv; kMaxBatch for the wide step)
+    int cap = 0;  // sequences the buffers hold
     pocr_seq *seq[kMaxBatch] = {};
     float *h = nullptr, *v = nullptr, *qkv = nullptr, *ho = nullptr, *g = nullptr;
     StepState *pad = nullptr;  // step state of the padding vectors
@@ -2889,8 +2888,8 @@ struct DecodeBatch {
     // partial Σx² of the hidden rows
     uint16_t *img = nullptr;
     float *ssq = nullptr;
-    bool rows_ok[2] = {false, false};  // more than kMaxNV rows, at most
-    float *logits = nullptr;  // [16][vocab] greedy rows of the MFMA LM head (vocab a multiple of 16)
+    bool rows_ok = false;
+    float *logits = nullptr;  // [16][vocab] greedy rows of the MFMA LM head (batch_small_head)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     bool owns = true;  // false: the vector buffers belong to a continuous batch
@@ -2902,16 +2901,14 @@ struct DecodeBatch {
                             (void *)xs, (void *)xb, (void *)rst, (void *)img, (void *)ssq, (void *)logits})
                 if (p) (void)hipFree(p);
     }
-    StepState *st(int i) const { return i < n ? seq[i]->st : pad; }
 };
 
-// states of the vectors base .. base+3 of a GEMV pass; vectors at or past lim
-// (padding, or rows outside the pass) take the dummy state
-GemvNV batch_nv(const DecodeBatch &b, int x_stride, int o_stride, int base = 0, int lim = kMaxBatch) {
+// the greedy rows base .. base+3 of a head pass over v; rows past the greedy
+// ones (padding) take the dummy state
+GemvNV batch_head_nv(const DecodeBatch &b, int base) {
     GemvNV q{};
-    q.x_stride = x_stride;
-    q.o_stride = o_stride;
-    for (int i = 1; i < kMaxNV; ++i) q.stv[i - 1] = base + i < lim ? b.st(base + i) : b.pad;
+    q.x_stride = b.m->cfg.hidden;
+    for (int i = 1; i < kMaxNV; ++i) q.stv[i - 1] = base + i < b.ng ? b.seq[base + i]->st : b.pad;
     return q;
 }
 
@@ -2968,18 +2965,23 @@ GemmParams batch_gemm(const DecodeBatch &b, const pocr_weight *w, int K) {
 }
 
 // The layers' weights all have tile images, the matrix kernels' only demand
-// (rows a multiple of 16, columns of 128).  Up to kMaxNV rows the shapes of the
-// streaming GEMV are asked for besides: the LM head's passes need them there,
-// and a step that takes other shapes is refused as a whole.
-bool batch_rows_ok(const pocr_model *m, bool narrow) {
+// (rows a multiple of 16, columns of 128).
+bool batch_rows_ok(const pocr_model *m) {
     for (const LayerW &L : m->layers) {
         for (const pocr_weight *w : L.w)
-            if (!w || !w->tiled || (narrow && !gemv_fast_shape(dev_mat(w)))) return false;
+            if (!w || !w->tiled) return false;
         if (L.w[POCR_W_Q]->qtype != L.w[POCR_W_K]->qtype || L.w[POCR_W_Q]->qtype != L.w[POCR_W_V]->qtype ||
             L.w[POCR_W_GATE]->qtype != L.w[POCR_W_UP]->qtype)
             return false;
     }
     return m->cfg.head_dim == kHD;
+}
+
+// Greedy rows whose head takes the small MFMA GEMM: more than one 4-vector pass
+// of them, or any that a multi-vector pass cannot take at all.
+bool batch_small_head(const pocr_model *m, int rows) {
+    if (rows < 2 || !m->lm || !gemm_small_ok(m->cfg.vocab, m->cfg.hidden)) return false;
+    return rows > kMaxNV || !gemv_fast_shape(dev_mat(m->lm));
 }
 
 // the batch's attention arguments of layer li
@@ -3093,7 +3095,7 @@ int enqueue_batch_step(DecodeBatch &b) {
         sb.tokens[i] = b.seq[i]->tokens;
         sb.max_tokens[i] = b.seq[i]->max_tokens;
     }
-    const bool rows = b.n > 1 && b.rows_ok[b.n <= kMaxNV];
+    const bool rows = b.n > 1 && b.rows_ok;
     hipLaunchKernelGGL(k_step_begin_multi, dim3(b.n), dim3(kThreads), 0, st, sb, m->embed, b.h, H, c.vocab, m->freq,
                        m->axis, m->layers[0].ln1, rows ? b.img : nullptr, b.n <= kRowsPackMax ? 1 : 0, b.ssq);
     HIP_TRY(hipGetLastError());
@@ -3102,8 +3104,6 @@ int enqueue_batch_step(DecodeBatch &b) {
     int rpw = 8, max_split = 1;
     for (int i = 0; i < b.n; ++i) rpw = std::max(rpw, b.seq[i]->rpw);
     for (int i = 0; i < b.n; ++i) max_split = std::max(max_split, attn_nsplit(b.seq[i]->cap, rpw));
-    const bool wide = b.n > kMaxNV;
-    if (wide && !rows) return fail(POCR_ERR_UNSUPPORTED, "batch step: %d rows need the weights' tile images", b.n);
     for (int li = 0; li < c.layers; ++li) {
         const LayerW &L = m->layers[li];
         const bool last = li + 1 == c.layers;
@@ -3111,61 +3111,65 @@ int enqueue_batch_step(DecodeBatch &b) {
             RC(batch_layer_rows(b, li, rpw, max_split));
             continue;
         }
-        // 1. RMSNorm(h)·ln1 → q|k|v for every sequence
-        GemvParams p{};
-        p.m[0] = dev_mat(L.w[POCR_W_Q]);
-        p.m[1] = dev_mat(L.w[POCR_W_K]);
-        p.m[2] = dev_mat(L.w[POCR_W_V]);
-        p.seg_end[0] = Q;
-        p.seg_end[1] = Q + KV;
-        p.seg_end[2] = QKV;
-        p.rows = QKV;
-        p.cols = H;
-        p.x = b.h;
-        p.norm_w = L.ln1;
-        p.eps = eps;
-        p.out = b.qkv;
-        p.st = b.st(0);
-        GemvNV q = batch_nv(b, H, QKV);
-        RC(gemv_launch(st, p, 1, PRO_RMSNORM, EPI_PLAIN, kBigGrid, b.nv, &q));
-        // 2. per sequence: RoPE + KV append + split attention, then the merge
+        // one sequence, or matrices without tile images: the single-vector GEMV
+        // for each sequence in turn
+        // 1. RMSNorm(h)·ln1 → q|k|v
+        for (int i = 0; i < b.n; ++i) {
+            GemvParams p{};
+            p.m[0] = dev_mat(L.w[POCR_W_Q]);
+            p.m[1] = dev_mat(L.w[POCR_W_K]);
+            p.m[2] = dev_mat(L.w[POCR_W_V]);
+            p.seg_end[0] = Q;
+            p.seg_end[1] = Q + KV;
+            p.seg_end[2] = QKV;
+            p.rows = QKV;
+            p.cols = H;
+            p.x = b.h + (size_t)i * H;
+            p.norm_w = L.ln1;
+            p.eps = eps;
+            p.out = b.qkv + (size_t)i * QKV;
+            p.st = b.seq[i]->st;
+            RC(gemv_launch(st, p, 1, PRO_RMSNORM, EPI_PLAIN, kBigGrid));
+        }
+        // 2. RoPE + KV append + split attention, then the merge
         RC(batch_attention(b, batch_attn(b, li, rpw, false), rpw, max_split));
-        // 3. o_proj + residual (+ the Q4/Q6 behaviour per sequence)
-        const pocr_weight *wo = L.w[POCR_W_O];
-        GemvParams o = gemv_params_1(wo);
-        o.x = b.ho;
-        o.residual = b.h;
-        o.vbuf = b.v;
-        o.st = b.st(0);
-        o.quirk = (m->quirk && (wo->qtype == POCR_Q4 || wo->qtype == POCR_Q6)) ? 1 : 0;
-        q = batch_nv(b, Q, H);
-        RC(gemv_launch(st, o, 1, PRO_COPY, EPI_OPROJ, kBigGrid, b.nv, &q));
-        // 4. RMSNorm(v)·ln2 → gate/up → SiLU(g)·u
-        GemvParams gu = gemv_params_1(L.w[POCR_W_GATE]);
-        gu.m[1] = dev_mat(L.w[POCR_W_UP]);
-        gu.x = b.v;
-        gu.norm_w = L.ln2;
-        gu.eps = eps;
-        gu.out = b.g;
-        gu.st = b.st(0);
-        q = batch_nv(b, H, F);
-        RC(gemv_launch(st, gu, 2, PRO_RMSNORM, EPI_SWIGLU, kBigGrid, b.nv, &q));
-        // 5. down + residual; last layer: v = h + down
-        GemvParams d = gemv_params_1(L.w[POCR_W_DOWN]);
-        d.x = b.g;
-        d.residual = b.h;
-        d.vbuf = b.v;
-        d.st = b.st(0);
-        d.flag = last ? 1 : 0;
-        q = batch_nv(b, F, H);
-        RC(gemv_launch(st, d, 1, PRO_COPY, EPI_DOWN, kBigGrid, b.nv, &q));
+        for (int i = 0; i < b.n; ++i) {
+            float *h = b.h + (size_t)i * H, *v = b.v + (size_t)i * H, *g = b.g + (size_t)i * F;
+            // 3. o_proj + residual (+ the Q4/Q6 behaviour)
+            const pocr_weight *wo = L.w[POCR_W_O];
+            GemvParams o = gemv_params_1(wo);
+            o.x = b.ho + (size_t)i * Q;
+            o.residual = h;
+            o.vbuf = v;
+            o.st = b.seq[i]->st;
+            o.quirk = (m->quirk && (wo->qtype == POCR_Q4 || wo->qtype == POCR_Q6)) ? 1 : 0;
+            RC(gemv_launch(st, o, 1, PRO_COPY, EPI_OPROJ, kBigGrid));
+            // 4. RMSNorm(v)·ln2 → gate/up → SiLU(g)·u
+            GemvParams gu = gemv_params_1(L.w[POCR_W_GATE]);
+            gu.m[1] = dev_mat(L.w[POCR_W_UP]);
+            gu.x = v;
+            gu.norm_w = L.ln2;
+            gu.eps = eps;
+            gu.out = g;
+            gu.st = b.seq[i]->st;
+            RC(gemv_launch(st, gu, 2, PRO_RMSNORM, EPI_SWIGLU, kBigGrid));
+            // 5. down + residual; last layer: v = h + down
+            GemvParams d = gemv_params_1(L.w[POCR_W_DOWN]);
+            d.x = g;
+            d.residual = h;
+            d.vbuf = v;
+            d.st = b.seq[i]->st;
+            d.flag = last ? 1 : 0;
+            RC(gemv_launch(st, d, 1, PRO_COPY, EPI_DOWN, kBigGrid));
+        }
     }
     // LM head on RMSNorm(v)·final_norm.  Greedy sequences: argmax into each
     // one's state — from kBatchWideHeadMin of them and a head the wide kernels
-    // take: one digit-plane launch and one 16-vector head for all; more than 4
-    // of them otherwise (and a vocabulary in 16-row blocks): digit planes, the
-    // small MFMA GEMM into logits rows and a per-row argmax; otherwise one GEMV
-    // pass per 4 of them (the last pass padded to 1, 2 or 4 vectors).
+    // take: one digit-plane launch and one 16-vector head for all; where
+    // batch_small_head says so: digit planes, the small MFMA GEMM into logits
+    // rows and a per-row argmax; otherwise one GEMV pass per 4 of them (the last
+    // pass padded to 1, 2 or 4 vectors), or per sequence where the head does not
+    // take several vectors.
     // Sampling sequences: each its own logits, top-k and draw (the draw lands
     // in argmax slot 0, where the next step reads it).
     const bool head_wide = b.ng >= kBatchWideHeadMin && b.xd && head_wide_ok(m->lm);
@@ -3174,7 +3178,7 @@ int enqueue_batch_step(DecodeBatch &b) {
         StepState *sts[kHeadWideVec];
         for (int i = 0; i < b.ng; ++i) sts[i] = b.seq[i]->st;
         RC(launch_head_wide(st, m->lm, b.v, H, b.ng, m->final_norm, eps, nullptr, 0, sts, b.xd, b.xs, b.xb));
-    } else if (wide && b.ng > kMaxNV && b.logits) {
+    } else if (b.logits && batch_small_head(m, b.ng)) {
         const int V = c.vocab;
         RC(batch_digitize(b, m->lm->qtype, b.v, H, m->final_norm));
         GemmParams lp = batch_gemm(b, m->lm, H);
@@ -3186,17 +3190,19 @@ int enqueue_batch_step(DecodeBatch &b) {
         hipLaunchKernelGGL(k_argmax_rows, dim3((V + kSlice - 1) / kSlice, b.ng), dim3(kThreads), 0, st, b.logits, V, V,
                            kSlice, b.rst);
         HIP_TRY(hipGetLastError());
-    }
-    for (int base = 0; base < b.ng && !head_wide && !(wide && b.ng > kMaxNV && b.logits); base += kMaxNV) {
-        const int left = b.ng - base;
-        const int nv = left == 1 ? 1 : (left == 2 ? 2 : 4);
-        GemvParams lm = gemv_params_1(m->lm);
-        lm.x = b.v + (size_t)base * H;
-        lm.norm_w = m->final_norm;
-        lm.eps = eps;
-        lm.st = b.st(base);
-        GemvNV q = batch_nv(b, H, 0, base, b.ng);
-        RC(gemv_launch(st, lm, 1, PRO_RMSNORM, EPI_ARGMAX, kBigGrid, nv, &q));
+    } else {
+        const int most = gemv_fast_shape(dev_mat(m->lm)) ? kMaxNV : 1;
+        for (int base = 0; base < b.ng; base += most) {
+            const int left = std::min(b.ng - base, most);
+            const int nv = left <= 2 ? left : 4;
+            GemvParams lm = gemv_params_1(m->lm);
+            lm.x = b.v + (size_t)base * H;
+            lm.norm_w = m->final_norm;
+            lm.eps = eps;
+            lm.st = b.seq[base]->st;
+            GemvNV q = batch_head_nv(b, base);
+            RC(gemv_launch(st, lm, 1, PRO_RMSNORM, EPI_ARGMAX, kBigGrid, nv, &q));
+        }
     }
     for (int i = b.ng; i < b.n; ++i) RC(enqueue_lm_head(b.seq[i], b.v + (size_t)i * H, false));
     return POCR_OK;
@@ -3220,14 +3226,14 @@ int32_t pending_token(const StepState &hs) {
     return (int32_t)(0xFFFFFFFFu - (uint32_t)(argmax_of(hs) & 0xFFFFFFFFull));
 }
 
-// vector buffers for b.cap rows; from kBatchWideHeadMin rows also the LM head's
-// digit planes (16 rows of the widest input); the operand images and row states
-// of batch_layer_rows
+// vector buffers for b.cap rows; for more than one also the LM head's digit
+// planes (16 rows of the widest input), the row states and the operand images of
+// batch_layer_rows
 int batch_alloc(DecodeBatch &b) {
     const pocr_config &c = b.m->cfg;
     const size_t H = c.hidden, Q = (size_t)c.heads * c.head_dim, KV = (size_t)c.kv_heads * c.head_dim;
     // whole GEMV passes: the head's last pass over 3 sequences reads 4 rows
-    const size_t rows = (std::max(b.cap, b.nv) + kMaxNV - 1) / kMaxNV * kMaxNV;
+    const size_t rows = (size_t)(b.cap + kMaxNV - 1) / kMaxNV * kMaxNV;
     hipStream_t s = b.m->ctx->stream;
     for (auto pr : {std::make_pair(&b.h, H), std::make_pair(&b.v, H), std::make_pair(&b.qkv, Q + 2 * KV),
                     std::make_pair(&b.ho, Q), std::make_pair(&b.g, (size_t)c.intermediate)}) {
@@ -3237,17 +3243,17 @@ int batch_alloc(DecodeBatch &b) {
     }
     HIP_TRY(hipMalloc(&b.pad, sizeof(StepState)));
     HIP_TRY(hipMemsetAsync(b.pad, 0, sizeof(StepState), s));
-    if (b.cap >= kBatchWideHeadMin) {
+    b.rows_ok = batch_rows_ok(b.m);
+    if (b.cap == 1) return POCR_OK;
+    {
         const size_t kmax = std::max(std::max(H, Q), (size_t)c.intermediate);
         HIP_TRY(hipMalloc(&b.xd, 3 * 16 * kmax));
         HIP_TRY(hipMemsetAsync(b.xd, 0, 3 * 16 * kmax, s));
         HIP_TRY(hipMalloc(&b.xs, 16 * sizeof(float)));
         HIP_TRY(hipMalloc(&b.xb, 16 * 4 * sizeof(int)));
     }
-    b.rows_ok[0] = batch_rows_ok(b.m, false);
-    b.rows_ok[1] = batch_rows_ok(b.m, true);
-    if (b.rows_ok[0] || b.cap > kMaxNV) HIP_TRY(hipMalloc(&b.rst, kMaxBatch * sizeof(StepState *)));
-    if (b.rows_ok[0]) {
+    HIP_TRY(hipMalloc(&b.rst, kMaxBatch * sizeof(StepState *)));
+    if (b.rows_ok) {
         // zeros: a row whose first step stops at once never writes its column
         const size_t img = rows_image_bytes((int)(H + Q) + c.intermediate), ssq = (H / 16) * 16 * sizeof(float);
         HIP_TRY(hipMalloc(&b.img, img));
@@ -3255,9 +3261,7 @@ int batch_alloc(DecodeBatch &b) {
         HIP_TRY(hipMalloc(&b.ssq, ssq));
         HIP_TRY(hipMemsetAsync(b.ssq, 0, ssq, s));
     }
-    if (b.cap > kMaxNV) {
-        if (gemm_small_ok(c.vocab, c.hidden)) HIP_TRY(hipMalloc(&b.logits, (size_t)16 * c.vocab * 4));
-    }
+    if (batch_small_head(b.m, b.cap)) HIP_TRY(hipMalloc(&b.logits, (size_t)16 * c.vocab * 4));
     return POCR_OK;
 }
 
@@ -3317,7 +3321,6 @@ extern "C" int pocr_decode_batch(pocr_seq *const *seqs, int n_seq, const int32_t
     b.n = n_seq;
     if (n_seq > batch_limit(m))
         return fail(POCR_ERR_UNSUPPORTED, "pocr_decode_batch: %d sequences need layer shapes the small GEMM takes", n_seq);
-    b.nv = n_seq == 1 ? 1 : (n_seq == 2 ? 2 : 4);
     b.cap = n_seq;
     batch_order(b, seqs, n_seq);
     RC(batch_alloc(b));
@@ -3428,7 +3431,6 @@ extern "C" int pocr_batch_create(pocr_model *m, pocr_batch **out) {
     b->m = m;
     b->bufs.m = m;
     b->limit = batch_limit(m);
-    b->bufs.nv = kMaxNV;
     b->bufs.cap = b->limit;
     const int rc = batch_alloc(b->bufs);
     if (rc == POCR_OK) {
@@ -3506,7 +3508,6 @@ static int batch_capture(pocr_batch *b) {
     for (auto &mb : b->members)
         if (!mb.finished) dec[nd++] = mb.s;
     batch_order(*d, dec, nd);
-    d->nv = d->n == 1 ? 1 : (d->n == 2 ? 2 : 4);
     d->cap = b->bufs.cap;
     d->h = b->bufs.h;
     d->v = b->bufs.v;
@@ -3520,7 +3521,7 @@ static int batch_capture(pocr_batch *b) {
     d->rst = b->bufs.rst;
     d->img = b->bufs.img;
     d->ssq = b->bufs.ssq;
-    std::copy(b->bufs.rows_ok, b->bufs.rows_ok + 2, d->rows_ok);
+    d->rows_ok = b->bufs.rows_ok;
     d->logits = b->bufs.logits;
     RC(batch_set_rows(*d));
     if (b->use_graph) {

@@ -29,6 +29,8 @@ SMALL = _cfg(512, 1280, 4, 2)
     (RAGGED, Q8, 2), (RAGGED, Q6, 3), (RAGGED, Q8, 4),   # (row, plane) columns
     (SMALL, Q4, 5), (SMALL, Q6, 5),                      # their last row
     (SMALL, Q4, 6), (SMALL, Q8, 8), (SMALL, Q6, 9),      # plane by plane; 8 rows a workgroup and the rest
+    # shapes the streaming GEMV does not take (down; the 4-bit head): small batches too
+    (SMALL, Q4, 2), (SMALL, Q8, 2), (SMALL, Q8, 3), (SMALL, Q6, 4),
     (SMALL, Q8, 16), (ERNIE, Q4, 3), (ERNIE, Q4, 9), (ERNIE, Q6, 16), (ERNIE, Q8, 2),
 ])
 def test_rows_match_single_decode(ctx, cfg, qtype, nseq):
@@ -71,3 +73,49 @@ def test_head_pass_over_the_last_three_rows(ctx, nseq):
         seqs.append((s, first))
     got = lib.decode_batch([s for s, _ in seqs], [f for _, f in seqs], [len(ids) for ids in prompts], 8, eos=())
     assert [list(g) for g in got] == want
+
+
+# matrices without tile images (520 columns): each sequence its own GEMVs
+UNTILED = _cfg(520, 1040, 4, 1)
+
+
+def _stream(m, ids, n_new):
+    """A prefilled sequence, its first token, and its stream decoded alone."""
+    s = m.seq(len(ids) + n_new + 4)
+    first = int(s.generate(ids, 1, eos=(), use_prefill=True)[0])
+    want = list(s.decode_greedy(first, len(ids), n_new, eos=()))
+    s.truncate(len(ids))
+    return s, first, want
+
+
+@pytest.mark.parametrize("nseq", [2, 3, 4])
+def test_batch_without_tile_images(ctx, nseq):
+    m = lib.Model(ctx, UNTILED)
+    m.load_weights(synth.make_weights(UNTILED, Q8, seed=35))
+    prompts = [synth.prompt_ids(1 + 3 * i, seed=700 + i, high=UNTILED.vocab) for i in range(nseq)]
+    seqs, firsts, want = zip(*[_stream(m, ids, 8) for ids in prompts])
+    got = lib.decode_batch(list(seqs), list(firsts), [len(ids) for ids in prompts], 8, eos=())
+    assert [list(g) for g in got] == list(want)
+
+
+@pytest.mark.parametrize("qtype,vocab", [(Q4, 1024), (Q4, 1000), (Q8, 1000)])
+def test_continuous_batch_drains(ctx, qtype, vocab):
+    # 6 members, then 4, 2 and 1, on shapes the streaming GEMV does not take; heads
+    # on the small GEMM, one pass per member, and 4-vector passes
+    cfg = DecoderConfig(hidden=512, inter=1280, layers=2, heads=4, kv_heads=2, head_dim=128, vocab=vocab, eps=1e-5,
+                        rope_theta=500000.0)
+    m = lib.Model(ctx, cfg)
+    m.load_weights(synth.make_weights(cfg, qtype, seed=34))
+    budgets = [4, 4, 9, 9, 14, 20]
+    prompts = [synth.prompt_ids(2 + 3 * i, seed=600 + i, high=vocab) for i in range(len(budgets))]
+    seqs, firsts, want = zip(*[_stream(m, ids, n) for ids, n in zip(prompts, budgets)])
+    b = lib.Batch(m)
+    for s, f, ids, n in zip(seqs, firsts, prompts, budgets):
+        b.join(s, f, len(ids), n, eos=())
+    left = [6]
+    while left[-1]:
+        left.append(b.step(20))
+    assert left == [6, 4, 2, 1, 0]
+    for s, w in zip(seqs, want):
+        assert list(b.leave(s)) == w
+    b.close()
