@@ -371,9 +371,8 @@ int pocr_decode_greedy(pocr_seq *s, int32_t first_token, int32_t first_pos, int 
  * first), out_counts[i] of them, stopping after an EOS id.  Greedy sequences
  * take the argmax, sampling ones (pocr_seq_set_sampling) draw from their own
  * generator.  Per-sequence results equal pocr_decode_greedy's up to f32
- * summation order.  Up to 4
- * sequences share GEMV passes; 5..16 need layer matrices with rows a
- * multiple of 16 and inputs a multiple of 256 (POCR_ERR_UNSUPPORTED
+ * summation order.  More than 4 sequences need layer matrices with rows a
+ * multiple of 16 and inputs a multiple of 128 (POCR_ERR_UNSUPPORTED
  * otherwise). */
 int pocr_decode_batch(pocr_seq *const *seqs, int n_seq, const int32_t *first_tokens,
                       const int32_t *first_positions, int max_new, const int32_t *eos, int n_eos,
@@ -382,7 +381,7 @@ int pocr_decode_batch(pocr_seq *const *seqs, int n_seq, const int32_t *first_tok
  * token steps, in place of the server's per-request slots, each running its
  * own decode loop (cmd/paddleocrvl-server/main.go:1106-1124, acquire/release;
  * model.go:1538-1568).  As many members decode at once as pocr_decode_batch
- * takes sequences (16, or 4 for models outside the wide step's shapes), one
+ * takes sequences (16, or 4 for models outside those shapes), one
  * batched device step per token; each member's tokens equal its
  * pocr_decode_greedy stream.  A batch is driven by one thread; a member
  * sequence accepts no other generation or cache call until it leaves

@@ -2923,16 +2923,14 @@ void batch_order(DecodeBatch &b, pocr_seq *const *seqs, int n) {
         if (seqs[i]->sampling) b.seq[b.n++] = seqs[i];
 }
 
-// Sequences a batch step can take: up to 4 on the GEMV passes, up to 16 when
-// every layer matrix fits the small MFMA GEMM (rows a multiple of 16, K a
-// multiple of 256).
+// Sequences a batch step can take: kMaxBatch where every layer matrix gets a tile
+// image at its upload, kMaxNV otherwise (each then costs a step of its own).
 int batch_limit(const pocr_model *m) {
     const pocr_config &c = m->cfg;
-    const int Q = c.heads * c.head_dim, KV = c.kv_heads * c.head_dim;
-    const bool wide = gemm_small_ok(Q + 2 * KV, c.hidden) && Q % 16 == 0 && KV % 16 == 0 &&
-                      gemm_small_ok(c.hidden, Q) && gemm_small_ok(c.intermediate, c.hidden) &&
-                      gemm_small_ok(c.hidden, c.intermediate);
-    return wide ? kMaxBatch : kMaxNV;
+    const int H = c.hidden, Q = c.heads * c.head_dim, KV = c.kv_heads * c.head_dim, F = c.intermediate;
+    const bool tiles = weight_tiles_ok(Q, H) && weight_tiles_ok(KV, H) && weight_tiles_ok(H, Q) &&
+                       weight_tiles_ok(F, H) && weight_tiles_ok(H, F);
+    return tiles ? kMaxBatch : kMaxNV;
 }
 
 // digit planes of the batch's n rows of x (RMSNorm·norm_w first if norm_w)
@@ -3320,7 +3318,7 @@ extern "C" int pocr_decode_batch(pocr_seq *const *seqs, int n_seq, const int32_t
     b.m = m;
     b.n = n_seq;
     if (n_seq > batch_limit(m))
-        return fail(POCR_ERR_UNSUPPORTED, "pocr_decode_batch: %d sequences need layer shapes the small GEMM takes", n_seq);
+        return fail(POCR_ERR_UNSUPPORTED, "pocr_decode_batch: %d sequences need layer rows in 16s and columns in 128s", n_seq);
     b.cap = n_seq;
     batch_order(b, seqs, n_seq);
     RC(batch_alloc(b));

@@ -23,6 +23,8 @@ ERNIE = _cfg(1024, 3072, 16, 2)
 RAGGED = _cfg(512, 1536, 4, 1)
 # 4 and 10 stages; 1,280 rows of gate and up
 SMALL = _cfg(512, 1280, 4, 2)
+# 5 and 33 stages: columns in 128s, not in 256s, and past the streaming GEMV's 4,096
+ODD = _cfg(640, 4224, 5, 1)
 
 
 @pytest.mark.parametrize("cfg,qtype,nseq", [
@@ -31,6 +33,7 @@ SMALL = _cfg(512, 1280, 4, 2)
     (SMALL, Q4, 6), (SMALL, Q8, 8), (SMALL, Q6, 9),      # plane by plane; 8 rows a workgroup and the rest
     # shapes the streaming GEMV does not take (down; the 4-bit head): small batches too
     (SMALL, Q4, 2), (SMALL, Q8, 2), (SMALL, Q8, 3), (SMALL, Q6, 4),
+    (ODD, Q4, 3), (ODD, Q6, 5), (ODD, Q4, 10), (ODD, Q8, 16),
     (SMALL, Q8, 16), (ERNIE, Q4, 3), (ERNIE, Q4, 9), (ERNIE, Q6, 16), (ERNIE, Q8, 2),
 ])
 def test_rows_match_single_decode(ctx, cfg, qtype, nseq):
