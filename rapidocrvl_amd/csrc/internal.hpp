@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <initializer_list>
 #include <memory>
 #include <mutex>
@@ -205,14 +206,16 @@ int download_staged(pocr_ctx *ctx, void *dst, const void *src, size_t bytes);
 // Transfers of a call whose operands are host arrays: the parts go through
 // pinned memory, the small ones with one copy kernel for all of them.
 // stage_in is stream-ordered (src may be reused at once); stage_out returns
-// with the bytes in place and the stream finished.
+// with the bytes in place and the stream finished.  accept, if given, runs once
+// the first (small) part is in place; an error from it leaves the others as they
+// were.
 struct HostPart {
     void *dst;
     const void *src;
     size_t bytes;  // a multiple of 4; 0: skipped
 };
 int stage_in(pocr_ctx *ctx, std::initializer_list<HostPart> parts);
-int stage_out(pocr_ctx *ctx, std::initializer_list<HostPart> parts);
+int stage_out(pocr_ctx *ctx, std::initializer_list<HostPart> parts, const std::function<int()> &accept = {});
 int batched_gemv(pocr_ctx *ctx, const DevMat &w, const float *x, int m, float *out);
 int read_state(pocr_seq *s, StepState *out);
 unsigned long long argmax_of(const StepState &s);

@@ -285,13 +285,15 @@ int pocr::stage_in(pocr_ctx *ctx, std::initializer_list<HostPart> parts) {
     return n ? launch_copy_parts(ctx, cp, n) : POCR_OK;
 }
 
-int pocr::stage_out(pocr_ctx *ctx, std::initializer_list<HostPart> parts) {
+int pocr::stage_out(pocr_ctx *ctx, std::initializer_list<HostPart> parts, const std::function<int()> &accept) {
     CopyParts cp{};
     int n = 0;
     size_t off = 0;
     if (parts.size() > kCopyParts) return fail(POCR_ERR_ARG, "stage_out: %zu parts", parts.size());
     RC(small_area(ctx, ctx->small_out, ctx->small_out_n, small_bytes(parts)));
+    bool large = false;
     for (const HostPart &h : parts) {
+        large = large || h.bytes > kSmallPart;
         if (!h.bytes || h.bytes > kSmallPart) continue;
         cp.src[n] = static_cast<const uint32_t *>(h.src);
         cp.dst[n] = reinterpret_cast<uint32_t *>(ctx->small_out + off);
@@ -300,17 +302,24 @@ int pocr::stage_out(pocr_ctx *ctx, std::initializer_list<HostPart> parts) {
     }
     if (n) RC(launch_copy_parts(ctx, cp, n));
     for (const HostPart &h : parts) {
-        if (h.bytes > kSmallPart) RC(download_staged(ctx, h.dst, h.src, h.bytes));
-        else if (h.bytes) touch_pages(h.dst, h.bytes);
+        if (h.bytes <= kSmallPart) touch_pages(h.dst, h.bytes);
+        else if (!accept) RC(download_staged(ctx, h.dst, h.src, h.bytes));
     }
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->in_used = 0;
     off = 0;
+    bool first = true;
     for (const HostPart &h : parts) {
-        if (!h.bytes || h.bytes > kSmallPart) continue;
-        std::memcpy(h.dst, ctx->small_out + off, h.bytes);
-        off += pad256(h.bytes);
+        if (h.bytes && h.bytes <= kSmallPart) {
+            std::memcpy(h.dst, ctx->small_out + off, h.bytes);
+            off += pad256(h.bytes);
+        }
+        if (first && accept) RC(accept());
+        first = false;
     }
+    if (!large || !accept) return POCR_OK;
+    for (const HostPart &h : parts)
+        if (h.bytes > kSmallPart) RC(download_staged(ctx, h.dst, h.src, h.bytes));
     return POCR_OK;
 }
 
@@ -2655,17 +2664,16 @@ int pocr::step_locked(pocr_seq *s, const float *emb, const int32_t pos3[3], int 
     RC(enqueue_step(s, 0, need_logits != 0, logits != nullptr));
     StepState hs;
     const bool out = need_logits && logits;
-    RC(stage_out(m->ctx, {{&hs, s->st, sizeof(StepState)}, {logits, s->logits, out ? (size_t)m->cfg.vocab * 4 : 0}}));
-    if (hs.err) return fail(POCR_ERR_DEVICE, "step: device state error %d", hs.err);
-    s->len = hs.len;
-    if (need_logits) {
-        if (token) {
+    return stage_out(m->ctx, {{&hs, s->st, sizeof(StepState)}, {logits, s->logits, out ? (size_t)m->cfg.vocab * 4 : 0}}, [&] {
+        if (hs.err) return fail(POCR_ERR_DEVICE, "step: device state error %d", hs.err);
+        s->len = hs.len;
+        if (need_logits && token) {
             const unsigned long long key = argmax_of(hs);
             if (key == 0ull) return fail(POCR_ERR_DEVICE, "step: no finite logit");
             *token = (int32_t)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFull));
         }
-    }
-    return POCR_OK;
+        return (int)POCR_OK;
+    });
 }
 
 extern "C" int pocr_step(pocr_seq *s, const float *emb, const int32_t pos3[3], int need_logits, float *logits,

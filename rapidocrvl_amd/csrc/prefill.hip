@@ -528,14 +528,15 @@ int prefill_run(pocr_seq *s, int n, const int32_t *pos3, float *logits, int32_t 
     RC(stage_in(m->ctx, {{s->st, &hs, sizeof(hs)}}));
     RC(enqueue_lm_head(s, b.v + (size_t)(n - 1) * H, logits != nullptr));
     StepState out;
-    RC(stage_out(m->ctx, {{&out, s->st, sizeof(out)}, {logits, s->logits, logits ? (size_t)c.vocab * 4 : 0}}));
-    s->len = clen0 + n;
-    if (token) {
-        const unsigned long long key = argmax_of(out);
-        if (key == 0ull) return fail(POCR_ERR_DEVICE, "prefill: no finite logit");
-        *token = (int32_t)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFull));
-    }
-    return POCR_OK;
+    return stage_out(m->ctx, {{&out, s->st, sizeof(out)}, {logits, s->logits, logits ? (size_t)c.vocab * 4 : 0}}, [&] {
+        s->len = clen0 + n;
+        if (token) {
+            const unsigned long long key = argmax_of(out);
+            if (key == 0ull) return fail(POCR_ERR_DEVICE, "prefill: no finite logit");
+            *token = (int32_t)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFull));
+        }
+        return (int)POCR_OK;
+    });
 }
 
 }  // namespace

@@ -374,3 +374,26 @@ def test_graph_replay_equals_direct_launches(ctx, monkeypatch):
     for (gk, gv), (dk, dv) in zip(g_kv, d_kv):
         assert np.array_equal(gk, dk) and np.array_equal(gv, dv)
     gm.close()
+
+
+@pytest.mark.parametrize("vocab", [300, 140000])  # logits beside the state, and in pieces of their own
+def test_failed_call_leaves_the_callers_logits(ctx, vocab):
+    # a head whose scales are NaN: no finite score, no token, no logits
+    cfg = DecoderConfig(hidden=128, inter=192, layers=1, heads=4, kv_heads=2, head_dim=128, vocab=vocab, eps=1e-5,
+                        rope_theta=500000.0)
+    w = synth.make_weights(cfg, Q8, seed=3)
+    qt, scales, packed, cols = w["lm_head"]
+    for head, fails in ((np.full_like(scales, np.nan), True), (scales, False)):
+        gm = lib.Model(ctx, cfg)
+        gm.load_weights({**w, "lm_head": (qt, head, packed, cols)})
+        s = gm.seq(8)
+        emb, pos = np.ascontiguousarray(w["embed"][:3]), np.array([[i, i, i] for i in range(3)], np.int32)
+        tok = np.zeros(1, np.int32)
+        n = lib.load()
+        for call in (lambda p: n.pocr_prefill(s.h, 3, emb.ctypes.data, pos.ctypes.data, p, tok.ctypes.data),
+                     lambda p: n.pocr_step(s.h, emb.ctypes.data, pos.ctypes.data, 1, p, tok.ctypes.data)):
+            logits = np.full(vocab, 7.0, np.float32)
+            assert (call(logits.ctypes.data) < 0) == fails
+            assert np.all(logits == 7.0) == fails
+        s.close()
+        gm.close()
