@@ -88,7 +88,7 @@ struct pocr_ctx {
     // pinned host memory of small transfers, each way; in_used bytes of the
     // former belong to copies that may still run
     uint8_t *small_in = nullptr, *small_out = nullptr;
-    size_t small_in_n = 0, small_out_n = 0, in_used = 0;
+    size_t in_used = 0;
     // pinned host read-back of the greedy decode loop: the step state and the
     // tokens of one batch of steps, fetched with one synchronization
     uint8_t *readback = nullptr;

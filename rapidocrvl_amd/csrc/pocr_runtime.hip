@@ -106,20 +106,13 @@ static int scratch_setup(int device, float **out) {
     return POCR_OK;
 }
 
-// an area of at least `bytes` (64 KB or a power of two; at most kCopyParts
-// parts' worth), grown with the stream idle
-static int small_area(pocr_ctx *ctx, uint8_t *&area, size_t &cap, size_t bytes) {
-    if (bytes <= cap) return POCR_OK;
-    size_t n = 64u << 10;
-    while (n < bytes) n *= 2;
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (area) (void)hipHostFree(area);
-    area = nullptr;
-    cap = 0;
-    HIP_TRY(hipHostMalloc((void **)&area, n, hipHostMallocDefault));
-    cap = n;
-    return POCR_OK;
-}
+// Small transfers (stage_in, stage_out): at most kCopyParts parts of at most
+// kSmallPart bytes a call.  Both areas hold a whole call's parts from the
+// context's creation on: none grows while a call waits for its results.
+constexpr int kCopyParts = 4;
+constexpr size_t kSmallPart = 512u << 10;
+constexpr size_t kSmallArea = kCopyParts * kSmallPart;
+
 extern "C" int pocr_ctx_create(int device, pocr_ctx **out) {
     if (!out) return fail(POCR_ERR_ARG, "pocr_ctx_create: null out");
     *out = nullptr;
@@ -141,12 +134,10 @@ extern "C" int pocr_ctx_create(int device, pocr_ctx **out) {
         delete c;
         return fail(POCR_ERR_DEVICE, "hipStreamCreate failed");
     }
-    // the first op-level call of a context would wait 25 µs for each of these
-    int rc = small_area(c, c->small_in, c->small_in_n, 1);
-    if (rc == POCR_OK) rc = small_area(c, c->small_out, c->small_out_n, 1);
-    if (rc != POCR_OK) {
+    if (hipHostMalloc((void **)&c->small_in, kSmallArea, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void **)&c->small_out, kSmallArea, hipHostMallocDefault) != hipSuccess) {
         ctx_release(c);
-        return rc;
+        return fail(POCR_ERR_NOMEM, "pocr_ctx_create: %zu bytes of pinned memory", 2 * kSmallArea);
     }
     *out = c;
     return POCR_OK;
@@ -230,8 +221,6 @@ int pocr::download_staged(pocr_ctx *ctx, void *dst, const void *src, size_t byte
 // Small parts: one kernel moves them between pinned host memory and their
 // places on the device (a copy call each costs the host 5-8 µs and a launch of
 // its own on the device).
-constexpr int kCopyParts = 4;
-constexpr size_t kSmallPart = 512u << 10;
 struct CopyParts {
     const uint32_t *src[kCopyParts];
     uint32_t *dst[kCopyParts];
@@ -253,21 +242,16 @@ static int launch_copy_parts(pocr_ctx *ctx, const CopyParts &cp, int parts) {
     return POCR_OK;
 }
 static size_t pad256(size_t b) { return (b + 255) / 256 * 256; }
-static size_t small_bytes(std::initializer_list<HostPart> parts) {
-    size_t b = 0;
-    for (const HostPart &h : parts) b += h.bytes <= kSmallPart ? pad256(h.bytes) : 0;
-    return b;
-}
 
 int pocr::stage_in(pocr_ctx *ctx, std::initializer_list<HostPart> parts) {
     CopyParts cp{};
     int n = 0;
     if (parts.size() > kCopyParts) return fail(POCR_ERR_ARG, "stage_in: %zu parts", parts.size());
-    const size_t need = small_bytes(parts);
-    if (ctx->in_used + need > ctx->small_in_n) {
+    size_t need = 0;
+    for (const HostPart &h : parts) need += h.bytes <= kSmallPart ? pad256(h.bytes) : 0;
+    if (ctx->in_used + need > kSmallArea) {
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         ctx->in_used = 0;
-        RC(small_area(ctx, ctx->small_in, ctx->small_in_n, need));
     }
     for (const HostPart &h : parts) {
         if (!h.bytes) continue;
@@ -290,7 +274,6 @@ int pocr::stage_out(pocr_ctx *ctx, std::initializer_list<HostPart> parts, const 
     int n = 0;
     size_t off = 0;
     if (parts.size() > kCopyParts) return fail(POCR_ERR_ARG, "stage_out: %zu parts", parts.size());
-    RC(small_area(ctx, ctx->small_out, ctx->small_out_n, small_bytes(parts)));
     bool large = false;
     for (const HostPart &h : parts) {
         large = large || h.bytes > kSmallPart;
