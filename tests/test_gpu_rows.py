@@ -1,7 +1,8 @@
 """The batched step's matrix kernels (2 to 16 rows over bf16 planes): the tokens
 and the K/V rows of a batched decode against each sequence decoded alone.  Both
 paths sum in f32 over exact products, about 1e-6 apart after three layers
-(2-norm); the bound is 2e-5."""
+(2-norm); the bound is 2e-5.  That does not see the third plane (dropping it
+moves sums by about 1e-6 too): test_all_bits_of_every_operand does."""
 import numpy as np
 import pytest
 
@@ -122,3 +123,61 @@ def test_continuous_batch_drains(ctx, qtype, vocab):
     for s, w in zip(seqs, want):
         assert list(b.leave(s)) == w
     b.close()
+
+
+def _one_hot(rows, cols, at, scale=1.0):
+    """A matrix that copies column at[r] to row r, exactly: code 1 times a power of two."""
+    codes = np.zeros((rows, cols), np.int8)
+    if at is not None:
+        codes[np.arange(rows), at] = 1
+    return Q8, np.full(rows, scale, np.float32), codes.view(np.uint8), cols
+
+
+def _bf16(x):
+    return synth.bf16_round(x)
+
+
+def _apart(a, b):
+    """Relative 2-norm distance up to a common factor (the norms' 1/rms)."""
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return np.linalg.norm(a / np.linalg.norm(a) - b / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("nseq", [2, 5, 6, 9, 16])  # (row, plane) columns; planes; 8 rows a workgroup and the rest
+def test_all_bits_of_every_operand(ctx, nseq):
+    """One step through matrices that copy columns: V of layer 0 is the embedding
+    row, V of layer 1 has gone through the attention merge, o_proj, gate/up and
+    down, each handing its values on as planes.  A value is rounded one to four
+    times on its way (about 3e-8 each, as a mean): the bound is 2e-7.  Without the
+    third plane, or with another row's, it is 2e-6 off."""
+    H, F, Q, KV = 512, 1280, 512, 256
+    rng = np.random.default_rng(nseq)
+    pick = lambda rows, cols: rng.permutation(np.resize(rng.permutation(cols), rows))
+    v0, o, up, down, v1 = pick(KV, H), pick(H, Q), pick(F, H), pick(H, F), pick(KV, H)
+    zero = {"q": _one_hot(Q, H, None), "k": _one_hot(KV, H, None), "o": _one_hot(H, Q, None),
+            "gate": _one_hot(F, H, None), "up": _one_hot(F, H, None), "down": _one_hot(H, F, None),
+            "ln1": np.ones(H, np.float32), "ln2": np.ones(H, np.float32)}
+    embed = rng.standard_normal((64, H)).astype(np.float32)
+    embed[:, 0] = 8.0  # every gate reads this column: one factor for all of a row
+    w = {"layers": [{**zero, "v": _one_hot(KV, H, v0), "o": _one_hot(H, Q, o),
+                     "gate": _one_hot(F, H, np.zeros(F, int)), "up": _one_hot(F, H, up),
+                     "down": _one_hot(H, F, down, 2.0 ** 30)},  # what down adds to is rounded away
+                    {**zero, "v": _one_hot(KV, H, v1)}],
+         "lm_head": _one_hot(64, H, pick(64, H)), "final_norm": np.ones(H, np.float32), "embed": embed}
+    m = lib.Model(ctx, DecoderConfig(hidden=H, inter=F, layers=2, heads=4, kv_heads=2, head_dim=128, vocab=64, eps=1e-5,
+                                     rope_theta=500000.0))
+    m.load_weights(w)
+    seqs = [m.seq(8) for _ in range(nseq)]
+    first = [3 * i + 1 for i in range(nseq)]
+    lib.decode_batch(seqs, first, [0] * nseq, 2, eos=())
+    for s, t in zip(seqs, first):
+        x = embed[t]
+        got0, got1 = s.read_kv(0)[1].reshape(-1), s.read_kv(1)[1].reshape(-1)
+        assert got0.size == KV and got1.size == KV
+        out = np.repeat(got0.reshape(2, 1, 128), 2, axis=1).reshape(-1)  # one cached row: both heads of a group give V
+        h1 = x + out[o]
+        want0, want1 = x[v0], h1[up[down[v1]]]
+        for got, want in ((got0, want0), (got1, want1)):
+            two = _bf16(want) + _bf16(want - _bf16(want))
+            assert _apart(two, want) > 6e-7
+            assert _apart(got, want) < 2e-7, (t, _apart(got, want))
