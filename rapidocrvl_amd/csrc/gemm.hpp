@@ -841,21 +841,15 @@ static __global__ void __launch_bounds__(kThreads) k_tile_weight(const uint8_t *
 template <int NPL>
 constexpr int kGemmStage = 2 * NPL * 2 * 64 * 16;
 
-// HBM → LDS load of BYTES (16 or 12) per lane: lane i's bytes land at
-// lds + 16·i.  Written as inline asm so the compiler's wait-count pass does
+// HBM → LDS load of 16 bytes per lane: lane i's bytes land at lds + 16·i.
+// Written as inline asm so the compiler's wait-count pass does
 // not see an LDS write it cannot place (it would wait for every load in flight
 // before each LDS read); the kernel orders these loads itself with wait_vm and
 // lds_barrier.
-template <int BYTES>
 __device__ __forceinline__ void lds_load(const void *g, void *lds) {
     const uint32_t base = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)lds);
-    if constexpr (BYTES == 16)
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(base)
-                     : "m0");
-    else
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx3 %0, off" ::"v"(g), "s"(base)
-                     : "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(base) : "m0");
 }
 
 // s_waitcnt vmcnt(N): at most N of this wave's vector-memory loads in flight
@@ -918,7 +912,7 @@ static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int 
     Raw raw0, raw1;
     auto issue = [&](int u, uint8_t *st, Raw &raw) {
 #pragma unroll
-        for (int i = 0; i < NPL; ++i) lds_load<16>(bsrc[i] + (size_t)4 * NPL * 1024 * u, st + boff[i]);
+        for (int i = 0; i < NPL; ++i) lds_load(bsrc[i] + (size_t)4 * NPL * 1024 * u, st + boff[i]);
 #pragma unroll
         for (int mi = 0; mi < NMAT; ++mi)
 #pragma unroll
@@ -1030,67 +1024,59 @@ static __global__ void __launch_bounds__(kThreads) k_gemm_lds(GemmParams p, int 
 }
 
 // ---------------------------------------------------------------------------
-// Small-M MFMA GEMM (M ≤ 16 tokens, the batched GEMV): a workgroup owns 16
-// rows (of each matrix with NMAT = 2) and all tokens; its 4 waves split K in
-// quarters, request their K-steps in double-buffered batches of four (a wave
-// waits on memory once or twice, not once per step), and their exact int32
-// partials are summed through LDS before wave 0 applies the epilogue.
+// Small-M MFMA GEMM (M ≤ 16 tokens: pocr_matvec, and batched LM heads that the
+// wide kernels do not take): a workgroup owns 16 rows and all tokens; its 4 waves
+// split K in quarters, request their K-steps in double-buffered batches of four
+// (a wave waits on memory once or twice, not once per step), and their exact
+// int32 partials are summed through LDS before wave 0 stores the rows.
 // ---------------------------------------------------------------------------
 constexpr int kSmallBatch = 4;  // K-steps per request batch
 
-template <int QT, int NMAT>
-static __global__ void __launch_bounds__(kThreads) k_gemm_small(GemmParams p, int epi) {
-    __shared__ v4i part[kWaves - 1][NMAT][3][64];
+template <int QT>
+static __global__ void __launch_bounds__(kThreads) k_gemm_small(GemmParams p) {
+    __shared__ v4i part[kWaves - 1][3][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r0 = blockIdx.x * 16;
     const int lr = lane & 15, lg = lane >> 4;
-    const GemmSeg sg = gemm_seg<NMAT>(p, r0);
+    const GemmSeg sg = gemm_seg<1>(p, r0);
     const int row_bytes = p.m[0].row_bytes;
-    const uint8_t *arow[NMAT];
-#pragma unroll
-    for (int mi = 0; mi < NMAT; ++mi) arow[mi] = sg.base[mi] + (size_t)(r0 + lr - sg.start) * row_bytes;
+    const uint8_t *arow = sg.base[0] + (size_t)(r0 + lr - sg.start) * row_bytes;
     const int8_t *brow = p.xd + (size_t)lr * p.K + 16 * lg;
     const int kq = p.K / kWaves;  // this wave's K range [wave·kq, (wave+1)·kq), a multiple of 64
     const int kbeg = wave * kq;
     const int nsteps = kq / kGemmK;
 
-    v4i acc[NMAT][3];
+    v4i acc[1][3];
 #pragma unroll
-    for (int mi = 0; mi < NMAT; ++mi)
-#pragma unroll
-        for (int pl = 0; pl < 3; ++pl) acc[mi][pl] = v4i{0, 0, 0, 0};
-    v4i a[kSmallBatch][NMAT], b[kSmallBatch][3];
-    auto load = [&](int s0, v4i (&aa)[kSmallBatch][NMAT], v4i (&bb)[kSmallBatch][3]) {
+    for (int pl = 0; pl < 3; ++pl) acc[0][pl] = v4i{0, 0, 0, 0};
+    v4i a[kSmallBatch], b[kSmallBatch][3];
+    auto load = [&](int s0, v4i (&aa)[kSmallBatch], v4i (&bb)[kSmallBatch][3]) {
 #pragma unroll
         for (int j = 0; j < kSmallBatch; ++j) {
             const int k0 = kbeg + kGemmK * min(s0 + j, nsteps - 1);  // clamped: loaded, not used
             const int k = k0 + 16 * lg;
-#pragma unroll
-            for (int mi = 0; mi < NMAT; ++mi) aa[j][mi] = load_codes16<QT>(arow[mi], k);
+            aa[j] = load_codes16<QT>(arow, k);
 #pragma unroll
             for (int pl = 0; pl < 3; ++pl) bb[j][pl] = *reinterpret_cast<const v4i *>(brow + pl * p.plane_stride + k0);
         }
     };
     load(0, a, b);
     for (int s0 = 0; s0 < nsteps; s0 += kSmallBatch) {
-        v4i an[kSmallBatch][NMAT], bn[kSmallBatch][3];
+        v4i an[kSmallBatch], bn[kSmallBatch][3];
         const bool more = s0 + kSmallBatch < nsteps;  // uniform
         if (more) load(s0 + kSmallBatch, an, bn);
 #pragma unroll
         for (int j = 0; j < kSmallBatch; ++j) {
             if (s0 + j >= nsteps) break;  // uniform
 #pragma unroll
-            for (int mi = 0; mi < NMAT; ++mi)
-#pragma unroll
-                for (int pl = 0; pl < 3; ++pl)
-                    acc[mi][pl] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j][mi], b[j][pl], acc[mi][pl], 0, 0, 0);
+            for (int pl = 0; pl < 3; ++pl)
+                acc[0][pl] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], b[j][pl], acc[0][pl], 0, 0, 0);
         }
         if (more) {
 #pragma unroll
             for (int j = 0; j < kSmallBatch; ++j) {
-#pragma unroll
-                for (int mi = 0; mi < NMAT; ++mi) a[j][mi] = an[j][mi];
+                a[j] = an[j];
 #pragma unroll
                 for (int pl = 0; pl < 3; ++pl) b[j][pl] = bn[j][pl];
             }
@@ -1098,23 +1084,19 @@ static __global__ void __launch_bounds__(kThreads) k_gemm_small(GemmParams p, in
     }
     if (wave > 0) {
 #pragma unroll
-        for (int mi = 0; mi < NMAT; ++mi)
-#pragma unroll
-            for (int pl = 0; pl < 3; ++pl) part[wave - 1][mi][pl][lane] = acc[mi][pl];
+        for (int pl = 0; pl < 3; ++pl) part[wave - 1][pl][lane] = acc[0][pl];
     }
     __syncthreads();
     if (wave > 0) return;
 #pragma unroll
     for (int w = 0; w < kWaves - 1; ++w)
 #pragma unroll
-        for (int mi = 0; mi < NMAT; ++mi)
-#pragma unroll
-            for (int pl = 0; pl < 3; ++pl) acc[mi][pl] += part[w][mi][pl][lane];
+        for (int pl = 0; pl < 3; ++pl) acc[0][pl] += part[w][pl][lane];
     const int n = lr;  // token (column)
     if (n >= p.ntok) return;
     const int rr = r0 + 4 * lg;
-    const float *const scl[2] = {sg.scale[0] + (rr - sg.start), NMAT == 2 ? sg.scale[1] + (rr - sg.start) : nullptr};
-    gemm_store<QT, NMAT>(p, epi, n, rr, scl, acc);
+    const float *const scl[2] = {sg.scale[0] + (rr - sg.start), nullptr};
+    gemm_store<QT, 1>(p, G_PLAIN, n, rr, scl, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1343,7 +1325,7 @@ static __global__ void __launch_bounds__(kPfThreads, 2) k_attn_prefill(const flo
         for (int i = 0; i < LPB; ++i) {
             const int piece = wave * LPB + i;
             const int blk = piece < kHalf / 1024 ? b0 : b1;
-            lds_load<16>(gimg + (size_t)blk * kPfImage + which * kHalf + (piece & (kHalf / 1024 - 1)) * 1024,
+            lds_load(gimg + (size_t)blk * kPfImage + which * kHalf + (piece & (kHalf / 1024 - 1)) * 1024,
                          buf + piece * 1024);
         }
     };
@@ -1567,7 +1549,7 @@ static __global__ void __launch_bounds__(kPfPairThreads) k_attn_prefill_pair(con
 #pragma unroll
         for (int i = 0; i < LPS; ++i) {
             const int chunk = wave * LPS + i;  // 1 KB chunk of the stage
-            if (two || chunk < kPfImage / 1024) lds_load<16>(src + 1024 * i, st + chunk * 1024);
+            if (two || chunk < kPfImage / 1024) lds_load(src + 1024 * i, st + chunk * 1024);
         }
     };
 

@@ -256,7 +256,7 @@ int tile_weight(hipStream_t s, int qtype, const uint8_t *src, int row_bytes, int
 int row_usum(hipStream_t s, int qtype, const uint8_t *src, int row_bytes, int rows, int cols, int *dst);
 // the small MFMA GEMM over at most 16 rows (digit planes of 16 rows)
 bool gemm_small_ok(int rows, int K);
-int gemm_small_rows(hipStream_t s, int qtype, const GemmParams &p, int epi);
+int gemm_small_rows(hipStream_t s, int qtype, const GemmParams &p);
 // a layer matrix of the batched decode step over operand images (rows.hip)
 struct RowsParams;
 int rows_gemm(hipStream_t s, int qtype, int epi, const RowsParams &p);

@@ -495,13 +495,13 @@ static bool pick_big(int tag, bool one, int lpr, int cpl, const void **fn) {
                     : gemv_fast_kernel<QT, 1, kBigU, 0, false>(lpr, cpl, fn);
 }
 
-// NV activation vectors per weight pass (batched decode): the big launch keeps
+// NV activation vectors per weight pass (one matrix): the big launch keeps
 // kBigU rows per lane group (U·NV ≤ 32 reduce-scatter entries, the workgroup
 // count and its activation prologues as for one vector) and gives every wave
 // one group
 template <int QT, int NV>
 static bool pick_nv(int nmat, int u, int lpr, int cpl, const void **fn) {
-    if (nmat == 2) return gemv_fast_kernel<QT, 2, 2, 0, false, 3, NV>(lpr, cpl, fn);
+    if (nmat == 2) return false;
     if (u == kBigU) return gemv_fast_kernel<QT, 1, kBigU, 0, true, 3, NV>(lpr, cpl, fn);
     if (u == 1) {  // only the down projection's shape takes one row per lane group here
         if (lpr != 32 || cpl != 3) return false;
@@ -2867,9 +2867,8 @@ struct DecodeBatch {
     pocr_seq *seq[kMaxBatch] = {};
     float *h = nullptr, *v = nullptr, *qkv = nullptr, *ho = nullptr, *g = nullptr;
     StepState *pad = nullptr;  // step state of the padding vectors
-    // digit planes of 16 rows, row scales and sums of the LM head (from
-    // kBatchWideHeadMin rows), and the rows' step states (the o_proj epilogue
-    // reads each sequence's clen)
+    // digit planes of 16 rows, row scales and sums of the LM head, and the rows'
+    // step states (the o_proj epilogue reads each sequence's clen)
     int8_t *xd = nullptr;
     float *xs = nullptr;
     int *xb = nullptr;
@@ -3174,7 +3173,7 @@ int enqueue_batch_step(DecodeBatch &b) {
         lp.ntok = b.ng;
         lp.out = b.logits;
         lp.out_stride = V;
-        RC(gemm_small_rows(st, m->lm->qtype, lp, G_PLAIN));
+        RC(gemm_small_rows(st, m->lm->qtype, lp));
         constexpr int kSlice = 2048;
         hipLaunchKernelGGL(k_argmax_rows, dim3((V + kSlice - 1) / kSlice, b.ng), dim3(kThreads), 0, st, b.logits, V, V,
                            kSlice, b.rst);
@@ -3216,8 +3215,7 @@ int32_t pending_token(const StepState &hs) {
 }
 
 // vector buffers for b.cap rows; for more than one also the LM head's digit
-// planes (16 rows of the widest input), the row states and the operand images of
-// batch_layer_rows
+// planes (16 rows), the row states and the operand images of batch_layer_rows
 int batch_alloc(DecodeBatch &b) {
     const pocr_config &c = b.m->cfg;
     const size_t H = c.hidden, Q = (size_t)c.heads * c.head_dim, KV = (size_t)c.kv_heads * c.head_dim;
@@ -3234,13 +3232,11 @@ int batch_alloc(DecodeBatch &b) {
     HIP_TRY(hipMemsetAsync(b.pad, 0, sizeof(StepState), s));
     b.rows_ok = batch_rows_ok(b.m);
     if (b.cap == 1) return POCR_OK;
-    {
-        const size_t kmax = std::max(std::max(H, Q), (size_t)c.intermediate);
-        HIP_TRY(hipMalloc(&b.xd, 3 * 16 * kmax));
-        HIP_TRY(hipMemsetAsync(b.xd, 0, 3 * 16 * kmax, s));
-        HIP_TRY(hipMalloc(&b.xs, 16 * sizeof(float)));
-        HIP_TRY(hipMalloc(&b.xb, 16 * 4 * sizeof(int)));
-    }
+    const size_t planes = std::max(3 * 16 * H, b.m->lm ? head_wide_plane_bytes(b.m->lm) : 0);
+    HIP_TRY(hipMalloc(&b.xd, planes));
+    HIP_TRY(hipMemsetAsync(b.xd, 0, planes, s));
+    HIP_TRY(hipMalloc(&b.xs, 16 * sizeof(float)));
+    HIP_TRY(hipMalloc(&b.xb, 16 * 4 * sizeof(int)));
     HIP_TRY(hipMalloc(&b.rst, kMaxBatch * sizeof(StepState *)));
     if (b.rows_ok) {
         // zeros: a row whose first step stops at once never writes its column

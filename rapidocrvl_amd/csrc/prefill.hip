@@ -91,13 +91,12 @@ int launch_gemm_t(hipStream_t s, int qtype, const GemmParams &p, int epi, int np
 }
 
 // small M (≤ 16 tokens): 16-row workgroups whose waves split K
-template <int NMAT>
-int launch_gemm_small_t(hipStream_t s, int qtype, const GemmParams &p, int epi) {
+int launch_gemm_small(hipStream_t s, int qtype, const GemmParams &p) {
     const dim3 grid(p.rows / 16);
     switch (qtype) {
-    case QT_Q8: hipLaunchKernelGGL((k_gemm_small<QT_Q8, NMAT>), grid, dim3(kThreads), 0, s, p, epi); break;
-    case QT_Q4: hipLaunchKernelGGL((k_gemm_small<QT_Q4, NMAT>), grid, dim3(kThreads), 0, s, p, epi); break;
-    case QT_Q6: hipLaunchKernelGGL((k_gemm_small<QT_Q6, NMAT>), grid, dim3(kThreads), 0, s, p, epi); break;
+    case QT_Q8: hipLaunchKernelGGL(k_gemm_small<QT_Q8>, grid, dim3(kThreads), 0, s, p); break;
+    case QT_Q4: hipLaunchKernelGGL(k_gemm_small<QT_Q4>, grid, dim3(kThreads), 0, s, p); break;
+    case QT_Q6: hipLaunchKernelGGL(k_gemm_small<QT_Q6>, grid, dim3(kThreads), 0, s, p); break;
     default: return fail(POCR_ERR_UNSUPPORTED, "gemm: qtype %d", qtype);
     }
     HIP_TRY(hipGetLastError());
@@ -318,7 +317,7 @@ int batched_gemv(pocr_ctx *ctx, const DevMat &w, const float *x, int m, float *o
     p.ntok = m;
     p.out = out;
     p.out_stride = w.rows;
-    if (small) return launch_gemm_small_t<1>(s, w.qtype, p, G_PLAIN);
+    if (small) return launch_gemm_small(s, w.qtype, p);
     return launch_gemm(s, w.qtype, 1, p, G_PLAIN, npad);
 }
 
@@ -546,10 +545,10 @@ int gemm_rows(hipStream_t s, int qtype, int nmat, const GemmParams &p, int epi, 
     return launch_gemm(s, qtype, nmat, p, epi, npad);
 }
 bool gemm_small_ok(int rows, int K) { return small_shape_ok(rows, K); }
-int gemm_small_rows(hipStream_t s, int qtype, const GemmParams &p, int epi) {
+int gemm_small_rows(hipStream_t s, int qtype, const GemmParams &p) {
     if (p.ntok > 16 || !small_shape_ok(p.rows, p.K) || p.plane_stride != (size_t)16 * p.K)
         return fail(POCR_ERR_UNSUPPORTED, "gemm: %d tokens of %dx%d outside the small kernel", p.ntok, p.rows, p.K);
-    return launch_gemm_small_t<1>(s, qtype, p, epi);
+    return launch_gemm_small(s, qtype, p);
 }
 
 }  // namespace pocr
