@@ -795,8 +795,9 @@ __device__ __forceinline__ int2 xcd_tile() {
 // in about equal parts.  The weights used to pass through LDS too, which cost
 // most where their 12-byte (Q6) pieces met the banks: 2,403 tokens, Q6, µs,
 // through LDS → registers: gate/up 83.5 → 64.6, q|k|v 36.7 → 31.1, o_proj and
-// down (mean) 37.6 → 32.2; 1,345 tokens, Q4: 29.9 → 29.8, 15.9 → 15.7,
-// 18.0 → 17.2.
+// down (mean) 37.6 → 32.2, Q8 80.2 → 67.9, 27.5 → 24.5, 32.9 → 29.5; 1,345
+// tokens, Q4: 29.9 → 29.8, 15.9 → 15.7, 18.0 → 17.2, Q8 50.1 → 39.4,
+// 18.1 → 17.7, 18.3 → 17.6.
 //
 // Per stage and wave: B 3 loads (1 KB each: 12 per workgroup), A NMAT·RB (Q4) or
 // 2·NMAT·RB (Q8, Q6) loads.  One barrier per stage: at its top every wave has

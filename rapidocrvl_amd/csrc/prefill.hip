@@ -105,13 +105,14 @@ int launch_gemm_small(hipStream_t s, int qtype, const GemmParams &p) {
 
 bool small_shape_ok(int rows, int K) { return rows % 16 == 0 && K % (kGemmK * kWaves) == 0 && K <= kMaxCols; }
 
-// One, two or four 16-row blocks per wave (64, 128 or 256 rows of each matrix
-// per workgroup), two-slot ring.  These kernels are latency-bound: the more
-// workgroups share a CU, the better their loads and barriers overlap, so the
-// row tile shrinks until the grid holds about three workgroups per CU.
-// Measured on the MI355X at 1,345 tokens (Q4, µs; 256 / 128 / 64-row tiles):
-// QKV 2560×1024 15.3 / 14.1 / 15.2; o_proj 1024×2048 16.5 / 13.5 / 12.3;
-// down 1024×3072 22.0 / 18.5 / 16.4; gate/up 2×3072×1024 – / 28.0 / 23.0.
+// One or two 16-row blocks per wave (64 or 128 rows of each matrix per
+// workgroup).  Two halve the LDS reads of the digit planes per row, one gives
+// twice the workgroups, whose loads and barriers overlap better: two are taken
+// for one matrix where they still leave about three workgroups per CU.
+// Measured inside prompts (µs, 128 / 64 rows): QKV 2560×1024 at 1,345 tokens Q4
+// 15.6 / 17.0, Q6 20.1 / 20.0; at 2,403 tokens 22.2 / 25.7, 29.6 / 31.5; o_proj
+// and down (688 workgroups of 64 rows at 1,345 tokens, mean) 18.9 / 17.2,
+// gate/up 35.6 / 29.8.
 template <int NMAT, int RB>
 int launch_gemm_lds_rb(hipStream_t s, int qtype, const GemmParams &p, int epi, int npad) {
     const dim3 grid((p.rows + 64 * RB - 1) / (64 * RB), npad / 32);

@@ -4,8 +4,12 @@
 // Every row of activations is handed from kernel to kernel as three bf16
 // planes: hi = bf16(x), mid = bf16(x − hi), lo = bf16(x − hi − mid).  Eight
 // significant bits each, so the three hold all 24 of an f32 and nothing of x is
-// lost; the weight codes (|code| ≤ 127) are exact in bf16 too, so the products
-// are exact and only the f32 accumulation rounds.  Unlike digit planes they
+// lost for 0 and 2^-103 ≤ |x| < 2^128 − 2^119: below, the last bits fall under
+// bf16's smallest normal number, 2^-126; from there on bf16(x) is infinite and
+// the row NaN.  The weight codes (|code| ≤ 127) are exact in bf16 too, so the
+// products are exact and only the f32 accumulation rounds (digit planes: exact
+// int32 sums over 22-bit operands; error against 64-bit sums level at 4 rows,
+// 2.01e-6 → 2.05e-6, and 16, 5.77e-6 → 5.65e-6).  Unlike digit planes they
 // need no scale, hence no pass over the whole row: the producer of a value (the
 // step prologue, the attention merge, the epilogues below) writes its planes
 // at once, already multiplied by the next RMSNorm's weight, and adds its square
@@ -15,11 +19,13 @@
 //
 // Bound: latency (launch, one round trip for weights and operands, the LDS sum),
 // and at 16 rows a CU's L2 rate for the operand image.  Measured inside decode
-// steps, kernel trace, µs (digitizing launch + small int8 GEMM before → now):
-// 16 rows Q4, 1,345 rows of context each: q|k|v 4.4 + 5.2 → 4.6, o_proj
-// 4.7 + 9.0 → 5.4, gate/up 4.4 + 6.1 → 5.7, down 5.4 + 9.0 → 7.0; 4 rows Q6
-// (four-vector GEMV before): 7.9 → 4.0, 7.1 → 4.9, 9.1 → 5.1, 8.3 → 5.6.
-// A step of 16 requests of the whole 4-bit model 1.26 → 0.83 ms.
+// steps, kernel trace, µs (digitizing launch + small int8 GEMM before → now, two
+// boxes): 16 rows Q4, 1,345 rows of context each: q|k|v 4.4 + 5.2 → 4.3–4.8,
+// o_proj 4.7 + 9.0 → 5.0–5.5, gate/up 4.4 + 6.1 → 5.2–5.7, down 5.4 + 9.0 →
+// 6.2–7.0; 4 rows Q6 (four-vector GEMV before): 7.9 → 4.0–4.4, 7.1 → 4.9–5.1,
+// 9.1 → 5.1–5.5, 8.3 → 5.6–5.9.  The step prologue, which writes the first
+// image, 4.4 → 5.5 at 4 rows.  A step of 16 requests of the whole 4-bit model
+// 1.26 → 0.82 ms.
 //
 // Operand image of K columns: for stage u (128 columns), plane and MFMA j the
 // 64 lanes' 16 bytes in lane order, lane (token n, group lg) holding columns

@@ -1,6 +1,6 @@
 """Batched greedy decode (pocr_decode_batch): several sequences of one model
-advance together — each layer GEMV streams its weights once for all of them,
-each sequence keeps its own KV cache.  Every sequence's stream must equal the
+advance together — each layer matrix is read once for all of them, each
+sequence keeps its own KV cache.  Every sequence's stream must equal the
 oracle's greedy stream for that sequence alone."""
 import numpy as np
 import pytest
@@ -124,8 +124,7 @@ def test_continuous_batch_staggered_joins(orc, ctx):
     assert b.step(2) == 3
     b.join(seqs[3][0], seqs[3][1], lens[3], budgets[3], eos=())
     assert b.step(1) == 4
-    # the fifth member moves the batch from the 4-vector GEMV passes to the
-    # wide (MFMA) step, and back once members finish
+    # the fifth member is the last on the matrix kernels' (row, plane) columns
     b.join(seqs[4][0], seqs[4][1], lens[4], budgets[4], eos=())
     pending = [0, 1, 2, 3, 4]
     for _ in range(100):
@@ -208,7 +207,7 @@ def test_continuous_batch_rules(ctx):
     other.close()
 
 
-# ---- wide batches: 5..16 sequences on the small MFMA GEMM ---------------------
+# ---- 5..16 sequences ----------------------------------------------------------
 
 @pytest.mark.parametrize("qtype,nseq", [(Q4, 5), (Q4, 8), (Q4, 16), (Q6, 16), (Q8, 11)],
                          ids=["q4-5", "q4-8", "q4-16", "q6-16", "q8-11"])
@@ -370,8 +369,8 @@ def test_continuous_batch_sampling_members(orc, ctx):
     b.close()
 
 
-# a vocabulary in 16-row blocks: more than 4 greedy rows take the MFMA LM head
-# (logits rows + per-row argmax) instead of the 4-vector GEMV passes
+# a vocabulary in 16-row blocks on the wide head, which takes 1,024 columns (the
+# small GEMM's head, logits rows + per-row argmax: test_gpu_rows.py, 512 columns)
 MID16 = DecoderConfig(hidden=1024, inter=3072, layers=3, heads=16, kv_heads=2, head_dim=128, vocab=5008, eps=1e-5,
                       rope_theta=500000.0)
 
