@@ -139,6 +139,8 @@ extern "C" int pocr_ctx_create(int device, pocr_ctx **out) {
         ctx_release(c);
         return fail(POCR_ERR_NOMEM, "pocr_ctx_create: %zu bytes of pinned memory", 2 * kSmallArea);
     }
+    // their pages touched here: a context's first small call 5 µs shorter
+    for (size_t off = 0; off < kSmallArea; off += 4096) c->small_in[off] = c->small_out[off] = 0;
     *out = c;
     return POCR_OK;
 }
