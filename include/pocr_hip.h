@@ -365,7 +365,7 @@ int pocr_decode_greedy(pocr_seq *s, int32_t first_token, int32_t first_pos, int 
 /* decode of n_seq (1..16) sequences of one model together: the
  * server's concurrent requests (cmd/paddleocrvl-server/main.go:1106, one
  * decode loop each, model.go:1538-1568) batched into one device step — each
- * layer's weights stream once for all of them (M = n_seq batched GEMV), each
+ * layer's weights stream once for all of them (M = n_seq rows), each
  * sequence keeps its own KV cache.  Sequence i starts from first_tokens[i] at
  * first_positions[i]; its tokens go to out_tokens[i*max_new ...] (first token
  * first), out_counts[i] of them, stopping after an EOS id.  Greedy sequences
